@@ -462,10 +462,10 @@ static bool run_mv1(Ctx* c, const JobSpec* js, int njobs, bool pair, const MvOpt
     return true;
 }
 
-// Several tokens: panel weights go to the int8-MFMA GEMM from kGemmMinTokens + 1 tokens (the
-// reference host's 16-token batches among them); otherwise (and for Q4_K / Q6_K) the general
-// matvec kernel runs over groups of at most HY_MAX_BATCH tokens. Both give every token the
-// single-token result. The threshold as measured (a fused_forward of the config-3 model, matvec
+// Several tokens: the int8-MFMA GEMM of the panel formats or of Q4_K / Q6_K from kGemmMinTokens + 1
+// tokens (the reference host's 16-token batches among them); below that, and for groups that mix
+// panels with the others, the general matvec kernel runs over groups of at most HY_MAX_BATCH
+// tokens. All give every token the single-token result. The threshold as measured on panels (a fused_forward of the config-3 model, matvec
 // against GEMM: 16 tokens 3.27 -> 1.95-2.01 ms, 8 tokens 2.34 -> 1.91-1.97, 4 tokens equal,
 // 2 tokens 1.71-1.78 against 1.87-1.92 ms)
 constexpr int kGemmMinTokens = 4;
@@ -484,7 +484,8 @@ static bool run_multi(Ctx* c, const JobSpec* js, int njobs, bool pair, int nt, c
             G.job[j].ldo = js[j].ldo;
             G.job[j].epi = js[j].epi;
         }
-        const hipError_t e = launch_gemm_panel(G, c->s);
+        hipError_t e = launch_gemm_panel(G, c->s);
+        if (e == hipErrorNotSupported) e = launch_gemm_kq(G, c->s);
         if (e != hipErrorNotSupported) {
             HIPCHK(c, e);
             return true;

@@ -1,0 +1,62 @@
+"""The Q4_K / Q6_K GEMM (k_gemm_kq) against the oracle, bit for bit.
+
+Cases sit at the edges of its tiles and splits: token counts around 16-token tiles and the counts
+where the split changes, row counts that end inside a 16-row tile, K from one block to past the
+largest that is split over wavefronts (33 blocks), and extreme block contents (every scale, min,
+code and activation at its largest magnitude, of either sign, where the int8 digits of the scaled
+weights and the f16 products of mins and bsums reach their bounds)."""
+import numpy as np
+import pytest
+
+from conftest import ROOT  # noqa: F401  (sys.path)
+from hymt2_amd import abi, synth
+from oracle import oracle as O
+from test_gpu_fallbacks import check_model
+from test_gpu_kernels import bits, run_matvec
+
+pytestmark = pytest.mark.gpu
+
+BLOCK = {abi.GT_Q4_K: 144, abi.GT_Q6_K: 210}
+
+
+def raw_weight(g, gt, n, k, extreme):
+    """Random block bytes (every code, scale and min value occurs); `extreme`: rows of constant
+    largest-magnitude fields. The f16 scales stay finite and of ordinary size."""
+    b = g.integers(0, 256, size=(n, k // 256, BLOCK[gt]), dtype=np.uint8)
+    if extreme:
+        b[0::3] = 0xFF               # Q4_K: q 15, sc 63, mn 63; Q6_K: q 31, sc -1
+        b[1::3] = 0x00               # Q6_K: q -32
+        if gt == abi.GT_Q6_K:
+            b[0::2, :, 192:208] = 0x80  # sc -128
+            b[1::2, :, 192:208] = 0x7F  # sc 127
+    d = synth.f16_bits(g.uniform(0.001, 0.02, size=(n, k // 256, 2))).view(np.uint8).reshape(n, k // 256, 4)
+    if gt == abi.GT_Q4_K:
+        b[:, :, 0:4] = d
+    else:
+        b[:, :, 208:210] = d[:, :, :2]
+    return synth.Weight(gt, k, n, b.reshape(n, -1))
+
+
+@pytest.mark.parametrize("gt", [abi.GT_Q4_K, abi.GT_Q6_K])
+@pytest.mark.parametrize("n,k", [(1, 256), (17, 512), (100, 2048), (63, 2304), (64, 3072), (65, 4096), (33, 4352),
+                                 (48, 6144), (31, 8192), (40, 8448), (4100, 512), (2200, 256)])
+def test_gemm_kq_vs_oracle(backend, gt, n, k):
+    g = synth.rng(gt * 13 + n + k)
+    for nt in (5, 16, 17, 48, 49, 80, 81, 128):
+        extreme = nt in (16, 49, 128)
+        w = raw_weight(g, gt, n, k, extreme)
+        x = synth.activations(g, nt, k)
+        if extreme:
+            x[0::2] = np.sign(x[0::2])  # every code 127 or -127
+            x[1::4] = 1.0               # and bsums at their largest
+        out, xq = run_matvec(backend, w, x)
+        assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, nt))), f"nt={nt}"
+
+
+def test_gemm_kq_in_a_model(backend):
+    """Mixed q/k (Q4_K) and v (Q6_K) rows in one launch, gate/up pairs with the SwiGLU epilogue and
+    residual adds, at the 1.8B layer's dimensions and batches that take every split of each."""
+    shape = synth.ModelShape(n_layer=1, hidden=2048, ffn=6144, heads=16, kv_heads=4, hdim=128, vocab=600, ctx=160)
+    model = synth.make_model(shape, mode="q4km", seed=171)
+    prompt = synth.rand_prompt(synth.rng(172), 150, shape.vocab)
+    check_model(backend, model, prompt, 4, batches=(16, 48, 77, 128), chunks=(16, 128))
