@@ -1251,9 +1251,9 @@ int hymt2_hip_gen_begin(void* impl, const hymt2_fused_args* shape, hy_dweight* e
     return gen_begin_at(c, shape, embd, vocab_out, prompt, n_prompt, n_total, 0, nullptr, 0);
 }
 
-// Whether the pipelined prefill applies: panel weights of the model's shapes in every layer
-// (the GEMM), gate and up pairable, hidden 2048 (its RMSNorm kernel) and the chunk attention
-// kernel with its fused Q8_K output.
+// Whether the pipelined prefill applies: weights of the model's shapes that the GEMMs take, each
+// launch's all of one of them (panels, or Q4_K / Q6_K), gate and up pairable, hidden 2048 (its
+// RMSNorm kernel) and the chunk attention kernel with its fused Q8_K output.
 static bool pipe_supported(const Fused* f, const hymt2_fused_args* a) {
     if (f->hidden != 2048) return false;
     AttnArgs at{};
@@ -1262,15 +1262,26 @@ static bool pipe_supported(const Fused* f, const hymt2_fused_args* a) {
     at.hdim = f->hdim;
     at.ctx = f->ctx;
     if (!attention_quantizes(at)) return false;
-    auto panel = [](const DW* w, int n, int k) { return w && w->mw.kind == KIND_PANEL && w->mw.n == n && w->mw.k == k; };
+    auto is = [](const DW* w, int n, int k) { return w && quant_kind(w->mw.kind) && w->mw.n == n && w->mw.k == k; };
+    auto panel = [](hy_dweight* w) { return dw(w)->mw.kind == KIND_PANEL; };
+    const hymt2_fused_layer& L0 = a->layers[0];
     for (int li = 0; li < a->n_layer; li++) {
         const hymt2_fused_layer& L = a->layers[li];
         const int H = f->hidden, F = f->ffn, Q = f->qdim, KV = f->kvdim;
-        if (!panel(dw(L.wq), Q, H) || !panel(dw(L.wk), KV, H) || !panel(dw(L.wv), KV, H) || !panel(dw(L.wo), H, Q) ||
-            !panel(dw(L.wg), F, H) || !panel(dw(L.wu), F, H) || !panel(dw(L.wd), H, F))
+        if (!is(dw(L.wq), Q, H) || !is(dw(L.wk), KV, H) || !is(dw(L.wv), KV, H) || !is(dw(L.wo), H, Q) ||
+            !is(dw(L.wg), F, H) || !is(dw(L.wu), F, H) || !is(dw(L.wd), H, F))
+            return false;
+        // a launch holds several layers' weights: one GEMM for all of them, and one kind of pairs
+        if (panel(L.wq) != panel(L0.wq) || panel(L.wk) != panel(L0.wq) || panel(L.wv) != panel(L0.wq) ||
+            panel(L.wo) != panel(L0.wo) || panel(L.wd) != panel(L0.wd) || dw(L.wg)->mw.kind != dw(L0.wg)->mw.kind ||
+            dw(L.wu)->mw.kind != dw(L0.wg)->mw.kind)
             return false;
     }
     return true;
+}
+
+static hipError_t launch_gemm(GemmPipeLaunch& L, hipStream_t s) {
+    return L.job[0].W.kind == KIND_PANEL ? launch_gemm_panel(L, s) : launch_gemm_kq(L, s);
 }
 
 static bool ensure_pipe(Ctx* c, Fused* f) {
@@ -1371,14 +1382,14 @@ static bool enqueue_prefill_pipe(Ctx* c, const hymt2_fused_args* a, int chunk, c
             pq.K = F;
             gu.pair = 1;
             HIPCHK(c, launch_rmsnorm_q8k(n1, rows, c->s));
-            HIPCHK(c, launch_gemm_panel(gq, c->s));
+            HIPCHK(c, launch_gemm(gq, c->s));
             HIPCHK(c, launch_rope_norm_store(pa, rows, c->s));
             HIPCHK(c, launch_attention(pa, rows, c->s));
-            HIPCHK(c, launch_gemm_panel(go, c->s));
+            HIPCHK(c, launch_gemm(go, c->s));
             HIPCHK(c, launch_rmsnorm_q8k(n2, rows, c->s));
-            HIPCHK(c, launch_gemm_panel(gu, c->s));
+            HIPCHK(c, launch_gemm(gu, c->s));
             HIPCHK(c, launch_quantize_q8k(pq, rows, c->s));
-            HIPCHK(c, launch_gemm_panel(gd, c->s));
+            HIPCHK(c, launch_gemm(gd, c->s));
         }
         if (g0 + m == nc) *h_last = f->p_h + (m - 1) * B * H + (size_t)(tokens(m - 1) - 1) * H;
     }

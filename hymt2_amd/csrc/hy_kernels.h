@@ -142,6 +142,7 @@ hipError_t launch_gemm_panel(GemmPipeLaunch& L, hipStream_t s);
 // The same for Q4_K and Q6_K weights (k_gemm_kq, hy_prefill_kq.hip), also mixed in one launch
 // (a pair's two of one kind); hipErrorNotSupported for any other kind.
 hipError_t launch_gemm_kq(GemmLaunch& L, hipStream_t s);
+hipError_t launch_gemm_kq(GemmPipeLaunch& L, hipStream_t s);
 
 struct AttnArgs {
     float* q;              // [nt][qdim]

@@ -528,6 +528,14 @@ hipError_t kq_shape(GemmLaunchT<NJ>& L, hipStream_t s) {
     for (int q = 0; q < L.njobs; q++)
         if (!PAIR || q % 2 == 0) rows += L.job[q].W.n;
     const int tt = (L.nt + 15) / 16;
+    if constexpr (NJ == kGemmPipeJobs) {
+        // several chunks: K whole; 4 token tiles a wavefront once their workgroups (64 rows by 64
+        // tokens) fill the chip, twice over for pairs. Two chunks of 128: pairs 37.8 us in 2 token
+        // tiles, 43.6 in 4; down 32.1 and 43.0. Eight: pairs 151 and 138, down 109 and 76, qkv 55 and 39
+        const int wgs = (rows + 63) / 64 * ((tt + 3) / 4);
+        if (tt >= 3 && wgs >= (PAIR ? 512 : 256)) return kq_go<Q, NJ, 4, 4, 1, 1, PAIR>(L, s);
+        return tt > 1 ? kq_go<Q, NJ, 2, 4, 1, 1, PAIR>(L, s) : kq_go<Q, NJ, 1, 4, 1, 1, PAIR>(L, s);
+    }
     if (L.nb <= 32 && (tt == 1 || (PAIR && tt <= 3 && L.nb <= 8))) return kq_split<Q, NJ, 1, 1, PAIR>(L, s);
     if constexpr (!PAIR)
         if (L.nb <= 32 && L.nb >= 12) return tt <= 3 ? kq_split<Q, NJ, 2, 1, false>(L, s) : kq_split<Q, NJ, 2, 2, false>(L, s);
@@ -569,5 +577,6 @@ hipError_t kq_dispatch(GemmLaunchT<NJ>& L, hipStream_t s) {
 }  // namespace
 
 hipError_t launch_gemm_kq(GemmLaunch& L, hipStream_t s) { return kq_dispatch(L, s); }
+hipError_t launch_gemm_kq(GemmPipeLaunch& L, hipStream_t s) { return kq_dispatch(L, s); }
 
 }  // namespace hy

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from conftest import ROOT  # noqa: F401  (sys.path)
-from hymt2_amd import abi, synth
+from hymt2_amd import abi, lib, synth
 from oracle import oracle as O
 from test_gpu_fallbacks import check_model
 from test_gpu_kernels import bits, run_matvec
@@ -60,3 +60,35 @@ def test_gemm_kq_in_a_model(backend):
     model = synth.make_model(shape, mode="q4km", seed=171)
     prompt = synth.rand_prompt(synth.rng(172), 150, shape.vocab)
     check_model(backend, model, prompt, 4, batches=(16, 48, 77, 128), chunks=(16, 128))
+
+
+@pytest.mark.parametrize("mode,odd", [("q4km", None), ("q4km", "up"), ("stq", "v"), ("q2", "down")])
+def test_pipelined_prefill_kinds(backend, mode, odd):
+    """The pipelined chunked prefill of Q4_K_M weights (3, 9 and 19 chunks, a ragged last one), and
+    models one of whose layers has a weight of another kind than its launch takes: `up` unlike its
+    gate, `v` unlike q and k, `down` unlike the other layers' (these run one chunk after another).
+    Greedy ids of the device loop, and the logits after them reading every layer's K/V."""
+    shape = synth.ModelShape(n_layer=3, hidden=2048, ffn=1024, heads=16, kv_heads=4, hdim=128, vocab=500, ctx=320)
+    model = synth.make_model(shape, mode=mode, seed=181)
+    g = synth.rng(182)
+    L = model["layers"][1]
+    if odd == "up":
+        L["wu"] = synth.make_weight(g, abi.GT_Q6_K, shape.ffn, shape.hidden)
+    elif odd == "v":
+        L["wv"] = synth.make_weight(g, abi.GT_Q6_K, shape.kvdim, shape.hidden)
+    elif odd == "down":
+        L["wd"] = synth.make_weight(g, abi.GT_Q4_K, shape.hidden, shape.ffn)
+    prompt = synth.rand_prompt(synth.rng(183), 290, shape.vocab)
+    want = O.OracleModel(model, threads=16).generate(prompt, 4, batch=16)
+    om = O.OracleModel(model, threads=16)
+    for i in range(0, len(prompt), 16):
+        om.forward(prompt[i:i + 16], i, want_logits=False)
+    ref = om.forward(want, len(prompt), want_logits=True)
+    fm = lib.FusedModel(backend, model)
+    try:
+        for chunk in (33, 128, 16):
+            ids, _ = fm.generate_device(prompt, 4, chunk=chunk)
+            assert np.array_equal(ids, want), f"chunk={chunk}"
+            assert np.array_equal(bits(fm.forward(list(ids), len(prompt), True)), bits(ref)), f"chunk={chunk}"
+    finally:
+        fm.close()
