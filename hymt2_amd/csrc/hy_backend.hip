@@ -131,6 +131,8 @@ struct Ctx {
     size_t act_cap = 0;
     float* out = nullptr;
     size_t out_cap = 0;
+    char* pin = nullptr;      // per-op staging of small groups (kPinBytes, pinned; kernels access it)
+    char* pin_dev = nullptr;  // its device address
     Fused* f = nullptr;
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     hipEvent_t ring[2] = {nullptr, nullptr};  // the last two decode launches of hymt2_hip_generate_ids
@@ -138,6 +140,13 @@ struct Ctx {
     int split_from = kSplitFromDefault;  // single-token attention at positions >= this: split form
     int pipe_depth = kPipeMax;           // chunks in flight in gen_prefill (1: one chunk after another)
 };
+
+// Per-op groups whose activations and outputs fit this go through pinned memory of the context: the
+// kernels write the outputs there over PCIe, and a copy kernel brings the activations to the device.
+// Copies to and from the caller's pageable buffers would each wait for the runtime's own staging
+// (a Q4_K gate/up group at one token: 47.5 us with them, 24.1 us without). Larger groups keep the
+// copies: their transfers are worth the DMA engine.
+constexpr size_t kPinBytes = 1u << 20;
 
 // Whether the single-token forward at position pos uses the split attention: long rows, and
 // every shape the one-kernel form (k_attn1: head dim 64 or 128, ctx <= kA1MaxCtx) does not take.
@@ -524,35 +533,83 @@ static bool ensure_scratch(Ctx* c, size_t act_bytes, size_t out_bytes) {
     return true;
 }
 
+static bool direct_out(const DW* w, const float* out, int nt) { return w->op_host && out == w->op_host && nt <= HY_MAX_BATCH; }
+
+// The group's contractions over the device activations act: each weight's output goes to its pinned
+// weight_out rows when the host passed those, else to its place in `out` (one after another).
+// Weights next to each other that one kernel takes share a launch (up to kMaxJobs).
+static bool matmul_launch(Ctx* c, hy_dweight* const* ws, float* const* outs, int cnt, int nt, const HyQ8K* act, float* out) {
+    auto panel = [&](int i) { return reinterpret_cast<const DW*>(ws[i])->mw.kind == KIND_PANEL; };
+    for (int i = 0; i < cnt;) {
+        JobSpec js[kMaxJobs];
+        int n = 0;
+        do {
+            const DW* w = reinterpret_cast<const DW*>(ws[i]);
+            const bool direct = direct_out(w, outs[i], nt);
+            js[n++] = JobSpec{w, direct ? w->op_dev : out, w->mw.n, EPI_STORE};
+            if (!direct) out += (size_t)w->mw.n * nt;
+            i++;
+        } while (i < cnt && n < kMaxJobs && panel(i) == panel(i - 1));
+        MvOpts o;
+        o.act = act;
+        if (!(nt == 1 ? run_mv1(c, js, n, false, o) : run_multi(c, js, n, false, nt, o))) {
+            c->broken = true;
+            return false;
+        }
+    }
+    return true;
+}
+
 // One per-op group on the given device staging: the host's Q8_K activations are copied to act,
-// each weight's output goes to its pinned weight_out rows when the host passed those (written by
-// the kernels directly), else to `out` and back to the host's buffer; one synchronisation.
+// outputs that do not go to weight_out rows to `out` and back to the host's buffers; one
+// synchronisation.
 static bool matmul_group(Ctx* c, hy_dweight* const* ws, float* const* outs, int cnt, const hymt2_q8k_block* xq, int nt,
                          HyQ8K* act, float* out) {
     const DW* w0 = reinterpret_cast<const DW*>(ws[0]);
     HIPCHK(c, hipMemcpyAsync(act, xq, (size_t)nt * w0->mw.nb * sizeof(HyQ8K), hipMemcpyHostToDevice, c->s));
-    size_t off = 0;
+    if (!matmul_launch(c, ws, outs, cnt, nt, act, out)) return false;
     for (int i = 0; i < cnt; i++) {
         const DW* w = reinterpret_cast<const DW*>(ws[i]);
-        const bool direct = w->op_host && outs[i] == w->op_host && nt <= HY_MAX_BATCH;
-        JobSpec j{w, direct ? w->op_dev : out + off, w->mw.n, EPI_STORE};
-        MvOpts o;
-        o.act = act;
-        if (!run_multi(c, &j, 1, false, nt, o)) {
-            c->broken = true;
-            return false;
-        }
-        if (!direct) off += (size_t)w->mw.n * nt;
-    }
-    off = 0;
-    for (int i = 0; i < cnt; i++) {
-        const DW* w = reinterpret_cast<const DW*>(ws[i]);
-        if (w->op_host && outs[i] == w->op_host && nt <= HY_MAX_BATCH) continue;
-        const size_t nbytes = (size_t)w->mw.n * nt * sizeof(float);
-        HIPCHK(c, hipMemcpyAsync(outs[i], out + off, nbytes, hipMemcpyDeviceToHost, c->s));
-        off += (size_t)w->mw.n * nt;
+        if (direct_out(w, outs[i], nt)) continue;
+        const size_t n = (size_t)w->mw.n * nt;
+        HIPCHK(c, hipMemcpyAsync(outs[i], out, n * sizeof(float), hipMemcpyDeviceToHost, c->s));
+        out += n;
     }
     HIPCHK(c, hipStreamSynchronize(c->s));
+    return true;
+}
+
+// The same through the context's pinned memory: abytes of activations, then the outputs.
+static bool matmul_group_pinned(Ctx* c, hy_dweight* const* ws, float* const* outs, int cnt, const hymt2_q8k_block* xq,
+                                int nt, size_t abytes) {
+    const DW* w0 = reinterpret_cast<const DW*>(ws[0]);
+    const size_t bytes = (size_t)nt * w0->mw.nb * sizeof(HyQ8K);
+    memcpy(c->pin, xq, bytes);
+    HIPCHK(c, launch_copy16(c->pin_dev, c->act, bytes, c->s));
+    if (!matmul_launch(c, ws, outs, cnt, nt, static_cast<HyQ8K*>(c->act), reinterpret_cast<float*>(c->pin_dev + abytes)))
+        return false;
+    HIPCHK(c, hipStreamSynchronize(c->s));
+    const char* from = c->pin + abytes;
+    for (int i = 0; i < cnt; i++) {
+        const DW* w = reinterpret_cast<const DW*>(ws[i]);
+        if (direct_out(w, outs[i], nt)) continue;
+        const size_t n = (size_t)w->mw.n * nt * sizeof(float);
+        memcpy(outs[i], from, n);
+        from += n;
+    }
+    return true;
+}
+
+static bool ensure_pin(Ctx* c) {
+    if (c->pin) return true;
+    void *p = nullptr, *pd = nullptr;
+    if (hipHostMalloc(&p, kPinBytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) return false;
+    if (hipHostGetDevicePointer(&pd, p, 0) != hipSuccess) {
+        (void)hipHostFree(p);
+        return false;
+    }
+    c->pin = static_cast<char*>(p);
+    c->pin_dev = static_cast<char*>(pd);
     return true;
 }
 
@@ -575,7 +632,7 @@ static size_t matmul_staging(Ctx* c, hy_dweight* const* ws, float* const* outs, 
             set_err(c, "matmul: weight %d unsupported for the per-op path", i);
             return 0;
         }
-        if (!(w->op_host && outs[i] == w->op_host && nt <= HY_MAX_BATCH)) out_total += (size_t)w->mw.n * nt;
+        if (!direct_out(w, outs[i], nt)) out_total += (size_t)w->mw.n * nt;
     }
     *act_bytes = ((size_t)nt * nb * sizeof(HyQ8K) + 255) / 256 * 256;
     return *act_bytes + out_total * sizeof(float);
@@ -586,7 +643,10 @@ static bool hip_matmul(void* impl, hy_dweight* const* ws, float* const* outs, in
     Ctx* c = static_cast<Ctx*>(impl);
     size_t abytes = 0;
     const size_t total = matmul_staging(c, ws, outs, cnt, xq, nt, &abytes);
-    if (!total || !ensure_scratch(c, abytes, total - abytes)) return false;
+    if (!total) return false;
+    if (total <= kPinBytes && ensure_pin(c))
+        return ensure_scratch(c, abytes, 0) && matmul_group_pinned(c, ws, outs, cnt, xq, nt, abytes);
+    if (!ensure_scratch(c, abytes, total - abytes)) return false;
     return matmul_group(c, ws, outs, cnt, xq, nt, static_cast<HyQ8K*>(c->act), c->out);
 }
 
@@ -1017,6 +1077,7 @@ static void hip_destroy_impl(void* impl) {
     free_fused(c->f);
     if (c->act) (void)hipFree(c->act);
     if (c->out) (void)hipFree(c->out);
+    if (c->pin) (void)hipHostFree(c->pin);
     for (hipEvent_t e : c->ev)
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->ring)
@@ -1061,6 +1122,7 @@ void* hymt2_hip_open(char* info, size_t cap) {
     for (hipEvent_t& e : c->ev) (void)hipEventCreate(&e);
     for (hipEvent_t& e : c->ring) (void)hipEventCreateWithFlags(&e, hipEventDisableTiming);
     c->scratch = scratch_address(c->dev);  // device 0 is current
+    (void)ensure_pin(c);  // (else matmul tries again, and copies)
     if (info && cap) snprintf(info, cap, "%s (%s, %d CUs)", prop.name[0] ? prop.name : "AMD GPU", prop.gcnArchName,
                               prop.multiProcessorCount);
     return c;

@@ -35,53 +35,42 @@ __device__ __forceinline__ void mv1_pin_job(const Mv1Job& J) {
     if (KIND == KIND_ANY) hy_sgpr_pin(J.W.kind);
 }
 
-// KIND: PANEL, Q4K, Q6K, or ANY (Q4K and Q6K jobs mixed; the kind is read per workgroup).
-// SPL: 16-byte segments per lane per row (the row has 32 * SPL segments).
+// The kernel's LDS (SPL 16-byte segments per lane per row, SPB per 256-weight block).
+template <int SPB, int SPL, int ITERS, int PRO>
+struct Mv1Lds {
+    static constexpr int NB = SPL * 32 / SPB;  // blocks per row
+    alignas(64) HyQ8K act[PRO == PRO_NONE ? 1 : NB];
+    float terms[kMv1Waves][2 * ITERS][NB];
+    typename std::conditional<PRO == PRO_NORM, HyExactLds, int>::type ex;  // of the norm only
+};
+
+// One workgroup's rows of job J (in pair mode of the gate J and the up weights UP): its weights'
+// kind KIND, so that the loads and terms are that kind's alone.
 template <int KIND, int SPL, int ITERS, int PRO>
-__global__ __launch_bounds__(kMv1Threads) void k_mv1(Mv1Launch L) {
+__device__ __forceinline__ void mv1_rows(Mv1Lds<KIND == KIND_PANEL ? 4 : 8, SPL, ITERS, PRO>& S, const Mv1Job& J,
+                                         const MvWeight& UP, bool pair, int rows_per_wg, const float* lx, const float* lnorm,
+                                         const HyQ8K* lact, float leps, unsigned long long* lslots, int n_arg) {
     constexpr int SPB = KIND == KIND_PANEL ? 4 : 8;  // segments per 256-weight block
     constexpr int NB = SPL * 32 / SPB;              // blocks per row
     constexpr int K = NB * HY_QK;
     constexpr int RPW = 2 * ITERS;                  // rows per wave
     static_assert(NB % (2 * kMv1Waves) == 0, "blocks per row must split in pairs over the waves");
-    __shared__ __align__(64) HyQ8K act_lds[PRO == PRO_NONE ? 1 : NB];
-    __shared__ float terms[kMv1Waves][RPW][NB];
-    using ExLds = typename std::conditional<PRO == PRO_NORM, HyExactLds, int>::type;  // LDS of the norm only
-    __shared__ ExLds ex_lds;
+    auto& act_lds = S.act;
+    auto& terms = S.terms;
+    auto& ex_lds = S.ex;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int hh = lane >> 5, j = lane & 31;
     const int wg = blockIdx.x;
-    // Every kernel argument this workgroup may use, loaded in one round of scalar loads and
-    // pinned in SGPRs before any selection: selecting the job by its index first makes the
-    // compiler load the chosen job's fields only once the index is known, several dependent
-    // round trips to memory before the first vector load can issue.
-    const Mv1Job j0 = L.job[0], j1 = L.job[1], j2 = L.job[2];
-    const int pair = L.pair, njobs = L.njobs, rows_per_wg = L.rows_per_wg;
-    const float* const lx = L.x;
-    const float* const lnorm = L.norm_w;
-    const HyQ8K* const lact = L.act;
-    const float leps = L.eps;
-    unsigned long long* const lslots = L.slots;
-    const int n_arg = L.n_arg;
-    hy_sgpr_pin(pair), hy_sgpr_pin(njobs), hy_sgpr_pin(rows_per_wg), hy_sgpr_pin(lx), hy_sgpr_pin(lnorm),
-        hy_sgpr_pin(lact), hy_sgpr_pin(leps), hy_sgpr_pin(lslots), hy_sgpr_pin(n_arg);
-    mv1_pin_job<KIND>(j0), mv1_pin_job<KIND>(j1), mv1_pin_job<KIND>(j2);
-    int jsel = 0;
-    if (!pair) {
-        if (njobs > 1 && wg >= j1.wg_begin) jsel = 1;
-        if (njobs > 2 && wg >= j2.wg_begin) jsel = 2;
-    }
-    const Mv1Job J = jsel == 0 ? j0 : (jsel == 1 ? j1 : j2);
+    constexpr int kind = KIND;
     const bool up = pair && hh;  // pair mode: half-wave 1 streams the up rows
-    const int kind = KIND == KIND_ANY ? J.W.kind : KIND;
-    const uint8_t* w = up ? j1.W.w : J.W.w;
-    const uint8_t* w2 = up ? j1.W.w2 : J.W.w2;
-    const int8_t* wsc = up ? j1.W.sc : J.W.sc;
-    const uint16_t* wdh = up ? j1.W.dh : J.W.dh;
-    const float* wps = up ? j1.W.ps : J.W.ps;
-    const int pshift = up ? j1.W.pshift : J.W.pshift;
-    const int poff = up ? j1.W.poff : J.W.poff;
+    const uint8_t* w = up ? UP.w : J.W.w;
+    const uint8_t* w2 = up ? UP.w2 : J.W.w2;
+    const int8_t* wsc = up ? UP.sc : J.W.sc;
+    const uint16_t* wdh = up ? UP.dh : J.W.dh;
+    const float* wps = up ? UP.ps : J.W.ps;
+    const int pshift = up ? UP.pshift : J.W.pshift;
+    const int poff = up ? UP.poff : J.W.poff;
     const int n = J.W.n;
     const int row0 = (wg - J.wg_begin) * rows_per_wg;
 
@@ -154,13 +143,7 @@ __global__ __launch_bounds__(kMv1Threads) void k_mv1(Mv1Launch L) {
 #pragma unroll
         for (int s = 0; s < SPL; s++) {
             const int f = j + 32 * s, b = f / SPB, sub = f % SPB;
-            float t;
-            if (KIND == KIND_ANY) {
-                t = kind == KIND_Q4K ? mv1_term<KIND_Q4K>(ws[i][s], A[s], sub, pshift, poff)
-                                     : mv1_term<KIND_Q6K>(ws[i][s], A[s], sub, pshift, poff);
-            } else {
-                t = mv1_term<KIND>(ws[i][s], A[s], sub, pshift, poff);
-            }
+            const float t = mv1_term<KIND>(ws[i][s], A[s], sub, pshift, poff);
             // every lane of the block holds the same term (its dot is reduced over the block's
             // lanes, its scales are the block's): an unconditional store, no exec-mask round trip
             terms[wave][rw][b] = t;
@@ -193,6 +176,48 @@ __global__ __launch_bounds__(kMv1Threads) void k_mv1(Mv1Launch L) {
             for (int b = 0; b < NB; b++) u += terms[wave][2 * lane + 1][b];
             J.out[p] = g / (1.0f + hy_expf(-g)) * u;  // SwiGLU, src/model.c:873-876
         }
+    }
+}
+
+// KIND: PANEL, Q4K, Q6K, or ANY (Q4K and Q6K jobs mixed: a workgroup branches once, on its job's
+// kind, to that kind's code; with the kind chosen at every load and term instead, a q/k/v launch of
+// 192 workgroups took 9.1 us in the decode graphs, 5.4 us now).
+template <int KIND, int SPL, int ITERS, int PRO>
+__global__ __launch_bounds__(kMv1Threads) void k_mv1(Mv1Launch L) {
+    __shared__ Mv1Lds<KIND == KIND_PANEL ? 4 : 8, SPL, ITERS, PRO> S;
+    const int wg = blockIdx.x;
+    // Every kernel argument this workgroup may use, loaded in one round of scalar loads and
+    // pinned in SGPRs before any selection: selecting the job by its index first makes the
+    // compiler load the chosen job's fields only once the index is known, several dependent
+    // round trips to memory before the first vector load can issue.
+    const Mv1Job j0 = L.job[0], j1 = L.job[1], j2 = L.job[2];
+    const int pair = L.pair, njobs = L.njobs, rows_per_wg = L.rows_per_wg;
+    const float* const lx = L.x;
+    const float* const lnorm = L.norm_w;
+    const HyQ8K* const lact = L.act;
+    const float leps = L.eps;
+    unsigned long long* const lslots = L.slots;
+    const int n_arg = L.n_arg;
+    // (one statement for the fields every kind reads: as several, the compiler may wait for the first
+    // ones' loads before it issues the others', a second round trip)
+    asm volatile("" ::"s"(pair), "s"(njobs), "s"(rows_per_wg), "s"(lx), "s"(lnorm), "s"(lact), "s"(leps), "s"(lslots),
+                 "s"(n_arg), "s"(j0.W.w), "s"(j0.W.n), "s"(j0.out), "s"(j0.epi), "s"(j0.wg_begin), "s"(j1.W.w), "s"(j1.W.n),
+                 "s"(j1.out), "s"(j1.epi), "s"(j1.wg_begin), "s"(j2.W.w), "s"(j2.W.n), "s"(j2.out), "s"(j2.epi),
+                 "s"(j2.wg_begin), "s"(j0.W.ps), "s"(j1.W.ps), "s"(j2.W.ps));
+    mv1_pin_job<KIND>(j0), mv1_pin_job<KIND>(j1), mv1_pin_job<KIND>(j2);
+    int jsel = 0;
+    if (!pair) {
+        if (njobs > 1 && wg >= j1.wg_begin) jsel = 1;
+        if (njobs > 2 && wg >= j2.wg_begin) jsel = 2;
+    }
+    const Mv1Job J = jsel == 0 ? j0 : (jsel == 1 ? j1 : j2);
+    if constexpr (KIND == KIND_ANY) {
+        if (J.W.kind == KIND_Q4K)
+            mv1_rows<KIND_Q4K, SPL, ITERS, PRO>(S, J, j1.W, pair, rows_per_wg, lx, lnorm, lact, leps, lslots, n_arg);
+        else
+            mv1_rows<KIND_Q6K, SPL, ITERS, PRO>(S, J, j1.W, pair, rows_per_wg, lx, lnorm, lact, leps, lslots, n_arg);
+    } else {
+        mv1_rows<KIND, SPL, ITERS, PRO>(S, J, j1.W, pair, rows_per_wg, lx, lnorm, lact, leps, lslots, n_arg);
     }
 }
 

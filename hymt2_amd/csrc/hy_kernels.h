@@ -286,6 +286,7 @@ inline bool embed_kind(int kind) {
 }
 hipError_t launch_embed(const int* ids, const int* step, const MvWeight& E, float* h, int H, hipStream_t s);
 hipError_t launch_embed_rows(const int* ids, int first, int nt, const MvWeight& E, float* h, int H, hipStream_t s);
+hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t s);  // multiples of 16 bytes
 hipError_t launch_set_int(int* p, int v, hipStream_t s);
 
 // The greedy argmax of v[0 .. n) as one key per 256-element workgroup into slots (argmax_grid(n) slots).

@@ -1599,6 +1599,17 @@ hipError_t launch_embed_rows(const int* ids, int first, int nt, const MvWeight& 
 
 __global__ void k_set_int(int* p, int v) { *p = v; }
 
+__global__ __launch_bounds__(256) void k_copy16(const uint4* src, uint4* dst, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t s) {
+    const size_t n = bytes / 16;
+    k_copy16<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(static_cast<const uint4*>(src), static_cast<uint4*>(dst), n);
+    return hipGetLastError();
+}
+
 hipError_t launch_set_int(int* p, int v, hipStream_t s) {
     k_set_int<<<1, 1, 0, s>>>(p, v);
     return hipGetLastError();
