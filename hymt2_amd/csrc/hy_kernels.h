@@ -114,7 +114,6 @@ struct GemmJob {
     float* out;
     int ldo;
     int epi;         // EPI_STORE / EPI_ADD
-    int tile_begin;  // first row tile of this job in the grid (set by the launcher)
     const HyQ8K* act;  // this job's activations [nt][nb] (null: the launch's act and nt)
     int nt;
 };
@@ -127,12 +126,77 @@ constexpr int kGemmPipeJobs = 3 * kPipeMax;
 template <int NJ>
 struct GemmLaunchT {
     GemmJob job[NJ];
+    int begin[NJ];         // first row tile of each job in the grid; kNoTile: none (set by the launcher)
     int njobs;
     int pair;              // jobs (2p, 2p + 1) = gate, up of equal shape: job[2p].out = silu(g) * u
     int nt;
     const HyQ8K* act;      // [nt][nb]
     int nb;                // set by the launcher
 };
+constexpr int kNoTile = 1 << 30;
+
+// The job of row tile wg (uniform), its first tile, and (PAIR) the up weights of a gate job. Every
+// field that the kernel reads is loaded in one round of scalar loads and pinned in SGPRs by one
+// statement: left to itself the compiler loads a chosen job's fields as it comes to them, five or
+// six dependent round trips before the first vector load. With three jobs all of them are loaded and
+// then selected; in a job table the begins are loaded first.
+#define HY_GEMM_REGS(J) "s"((J).W.w), "s"((J).W.n), "s"((J).out), "s"((J).ldo), "s"((J).epi), "s"((J).act), "s"((J).nt)
+#define HY_GEMM_PANEL_REGS(W) "s"((W).ps), "s"((W).pshift), "s"((W).poff)
+#define HY_GEMM_KQ_REGS(W) "s"((W).w2), "s"((W).sc), "s"((W).dh), "s"((W).kind)
+template <bool PANEL, bool PAIR, int NJ>
+__device__ __forceinline__ void gemm_job(const GemmLaunchT<NJ>& L, int wg, GemmJob& J, MvWeight& UP, int& begin, int& nb) {
+    nb = L.nb;
+    if constexpr (NJ == kMaxJobs) {
+        const GemmJob j0 = L.job[0], j1 = L.job[1], j2 = L.job[2];
+        const int b1 = L.begin[1], b2 = L.begin[2];
+        if constexpr (PANEL && PAIR)
+            asm volatile("" ::"s"(nb), HY_GEMM_REGS(j0), HY_GEMM_PANEL_REGS(j0.W), "s"(j1.W.w), HY_GEMM_PANEL_REGS(j1.W));
+        else if constexpr (PANEL)
+            asm volatile("" ::"s"(nb), "s"(b1), "s"(b2), HY_GEMM_REGS(j0), HY_GEMM_PANEL_REGS(j0.W), HY_GEMM_REGS(j1),
+                         HY_GEMM_PANEL_REGS(j1.W), HY_GEMM_REGS(j2), HY_GEMM_PANEL_REGS(j2.W));
+        else if constexpr (PAIR)
+            asm volatile("" ::"s"(nb), HY_GEMM_REGS(j0), HY_GEMM_KQ_REGS(j0.W), "s"(j1.W.w), HY_GEMM_KQ_REGS(j1.W));
+        else
+            asm volatile("" ::"s"(nb), "s"(b1), "s"(b2), HY_GEMM_REGS(j0), HY_GEMM_KQ_REGS(j0.W), HY_GEMM_REGS(j1),
+                         HY_GEMM_KQ_REGS(j1.W), HY_GEMM_REGS(j2), HY_GEMM_KQ_REGS(j2.W));
+        if (PAIR) {
+            J = j0, UP = j1.W, begin = 0;
+        } else {
+            J = wg >= b2 ? j2 : wg >= b1 ? j1 : j0;
+            begin = wg >= b2 ? b2 : wg >= b1 ? b1 : 0;
+        }
+    } else {
+        int j = 0;
+        begin = 0;
+#pragma unroll
+        for (int q = 1; q < NJ; q++) {
+            const int b = L.begin[q];
+            if (wg >= b) j = q, begin = b;
+        }
+        J = L.job[j];
+        if (PAIR) UP = L.job[j + 1].W;
+        if constexpr (PANEL && PAIR)
+            asm volatile("" ::"s"(nb), HY_GEMM_REGS(J), HY_GEMM_PANEL_REGS(J.W), "s"(UP.w), HY_GEMM_PANEL_REGS(UP));
+        else if constexpr (PANEL)
+            asm volatile("" ::"s"(nb), HY_GEMM_REGS(J), HY_GEMM_PANEL_REGS(J.W));
+        else if constexpr (PAIR)
+            asm volatile("" ::"s"(nb), HY_GEMM_REGS(J), HY_GEMM_KQ_REGS(J.W), "s"(UP.w), HY_GEMM_KQ_REGS(UP));
+        else
+            asm volatile("" ::"s"(nb), HY_GEMM_REGS(J), HY_GEMM_KQ_REGS(J.W));
+    }
+}
+// Sets a launch's begins for tiles of rows_wg rows (in pair mode the up jobs carry none); returns
+// the number of row tiles.
+template <int NJ>
+inline int gemm_tiles(GemmLaunchT<NJ>& L, int rows_wg) {
+    int tiles = 0;
+    for (int q = 0; q < NJ; q++) {
+        const bool own = q < L.njobs && !(L.pair && q % 2);
+        L.begin[q] = own ? tiles : kNoTile;
+        if (own) tiles += (L.job[q].W.n + rows_wg - 1) / rows_wg;
+    }
+    return tiles;
+}
 using GemmLaunch = GemmLaunchT<kMaxJobs>;
 using GemmPipeLaunch = GemmLaunchT<kGemmPipeJobs>;
 // hipErrorNotSupported for weights that are not panels of one K (the caller then uses

@@ -124,39 +124,35 @@ __global__ __launch_bounds__(kGemmThreads * KS) void k_gemm_panel(GemmLaunchT<NJ
     if (PAIR && tid < 32) etab[tid] = hy_exp_tab_entry(tid);  // read after the block barriers
     const int half = KS == 2 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;  // K set
     const int wr = wave % WR, wt = wave / WR;
-    const int nb = L.nb;
+    // job of this row tile (uniform; in pair mode only the gate jobs 2p carry tiles)
+    GemmJob J;
+    MvWeight UP{};
+    int begin, nb;
+    gemm_job<true, PAIR, NJ>(L, blockIdx.x, J, UP, begin, nb);
     const int nbh = KS == 2 ? NBH : nb;  // blocks of this K set, from block hb0
     const int hb0 = half * nbh;
-
-    // job of this row tile (uniform; in pair mode only the gate jobs 2p carry tiles)
-    int j = 0;
-#pragma unroll
-    for (int q = 1; q < NJ; q++)
-        if (q < L.njobs && (int)blockIdx.x >= L.job[q].tile_begin) j = q;
     const int rows_wg = PAIR ? WR * 16 : SLOTS;
-    const int row0 = ((int)blockIdx.x - L.job[j].tile_begin) * rows_wg;
+    const int row0 = ((int)blockIdx.x - begin) * rows_wg;
     const int tokw = (int)blockIdx.y * TOK;  // first token of the workgroup
-    const HyQ8K* const act = L.job[j].act;  // a pair's gate and up share their tokens
-    const int nt = L.job[j].nt;
+    const HyQ8K* const act = J.act;  // a pair's gate and up share their tokens
+    const int nt = J.nt;
     if (tokw >= nt) return;  // a shorter chunk of a pipelined launch (uniform)
 
-    auto slot_job = [&](int mt) { return PAIR ? j + mt : j; };
     // weight row of local row slot s = w_r * MT * 16 + mt * 16 + rr
     auto slot_row = [&](int w_r, int mt, int rr) {
         return PAIR ? row0 + w_r * 16 + rr : row0 + w_r * MT * 16 + mt * 16 + rr;
     };
 
-    // Per row tile: its weight (uniform; read from the kernel arguments with scalar loads: a
-    // per-lane index into the job table would turn every field into a dependent vector load).
+    // per row tile: its weight (uniform)
     const uint8_t* wbase[MT];
     const float* psbase[MT];
     int nrow[MT], psh[MT], pof[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-        const MvWeight& W = L.job[slot_job(mt)].W;
+        const MvWeight& W = PAIR && mt ? UP : J.W;
         wbase[mt] = W.w;
         psbase[mt] = W.ps;
-        nrow[mt] = W.n;
+        nrow[mt] = J.W.n;  // (a pair's are of equal rows)
         psh[mt] = W.pshift;
         pof[mt] = W.poff;
     }
@@ -340,8 +336,8 @@ __global__ __launch_bounds__(kGemmThreads * KS) void k_gemm_panel(GemmLaunchT<NJ
     }
 
     // epilogue: lane holds rows 4 g .. 4 g + 3 of each row tile for token tl of each token tile
-    float* const out = L.job[j].out;
-    const int ldo = L.job[j].ldo, nout = L.job[j].W.n, epi = L.job[j].epi;
+    float* const out = J.out;
+    const int ldo = J.ldo, nout = J.W.n, epi = J.epi;
 #pragma unroll
     for (int n = 0; n < NT; n++) {
         const int t = tokw + wt * NT * 16 + n * 16 + tl;
@@ -387,15 +383,7 @@ __global__ __launch_bounds__(kGemmThreads * KS) void k_gemm_panel(GemmLaunchT<NJ
 template <int NJ, int MT, int NT, int WR, int WT, bool PAIR, int RING, int KS = 1, int NBH = 0>
 hipError_t gemm_go(GemmLaunchT<NJ>& L, hipStream_t s) {
     const int rows_wg = PAIR ? WR * 16 : WR * MT * 16;
-    int tiles = 0;
-    for (int q = 0; q < L.njobs; q++) {
-        if (PAIR && q % 2) {
-            L.job[q].tile_begin = 1 << 30;  // an up job: never selected by tile index
-            continue;
-        }
-        L.job[q].tile_begin = tiles;
-        tiles += (L.job[q].W.n + rows_wg - 1) / rows_wg;
-    }
+    const int tiles = gemm_tiles(L, rows_wg);
     const int toks_wg = WT * NT * 16;
     const dim3 grid(tiles, (L.nt + toks_wg - 1) / toks_wg);
     k_gemm_panel<NJ, MT, NT, WR, WT, PAIR, RING, KS, NBH><<<grid, kGemmThreads * KS, 0, s>>>(L);

@@ -449,40 +449,16 @@ __device__ __forceinline__ void kq_tile(const GemmJob& J, const MvWeight& UP, in
 }
 
 // Q: the launch may hold Q4_K (bit 0) and Q6_K (bit 1) jobs.
-template <int Q>
-__device__ __forceinline__ void kq_pin(const GemmJob& J) {
-    hy_sgpr_pin(J.W.w), hy_sgpr_pin(J.W.n), hy_sgpr_pin(J.out), hy_sgpr_pin(J.ldo), hy_sgpr_pin(J.epi);
-    hy_sgpr_pin(J.tile_begin), hy_sgpr_pin(J.act), hy_sgpr_pin(J.nt);
-    if (Q & 2) hy_sgpr_pin(J.W.w2), hy_sgpr_pin(J.W.sc), hy_sgpr_pin(J.W.dh);
-    if (Q == 3) hy_sgpr_pin(J.W.kind);
-}
-
 template <int Q, int NJ, int NT, int W, int KS, int NBH, bool PAIR>
 __global__ __launch_bounds__(64 * W * KS) void k_gemm_kq(GemmLaunchT<NJ> L) {
     __shared__ KqLds<NT, W, KS> S;
-    if (PAIR && threadIdx.x < 32) S.etab[threadIdx.x] = hy_exp_tab_entry(threadIdx.x);  // read after the block barriers
-    const int wg = blockIdx.x, nb = L.nb, njobs = L.njobs;
     GemmJob J;
     MvWeight UP{};
-    if constexpr (NJ == kMaxJobs) {
-        // every job's fields in one round of scalar loads: selecting first makes them several
-        // dependent round trips before the first vector load
-        const GemmJob j0 = L.job[0], j1 = L.job[1], j2 = L.job[2];
-        hy_sgpr_pin(nb), hy_sgpr_pin(njobs);
-        kq_pin<Q>(j0), kq_pin<Q>(j1);
-        if (!PAIR) kq_pin<Q>(j2);
-        J = j0;
-        if (PAIR) UP = j1.W;
-        else J = njobs > 2 && wg >= j2.tile_begin ? j2 : njobs > 1 && wg >= j1.tile_begin ? j1 : j0;
-    } else {
-        int j = 0;
-#pragma unroll
-        for (int q = 1; q < NJ; q++)
-            if (q < njobs && wg >= L.job[q].tile_begin) j = q;
-        J = L.job[j];
-        if (PAIR) UP = L.job[j + 1].W;
-    }
-    const int row0 = (wg - J.tile_begin) * 16 * W, t0 = (int)blockIdx.y * 16 * NT;
+    int begin, nb;
+    const int wg = blockIdx.x;
+    gemm_job<false, PAIR, NJ>(L, wg, J, UP, begin, nb);
+    if (PAIR && threadIdx.x < 32) S.etab[threadIdx.x] = hy_exp_tab_entry(threadIdx.x);  // read after the block barriers
+    const int row0 = (wg - begin) * 16 * W, t0 = (int)blockIdx.y * 16 * NT;
     if (t0 >= J.nt) return;  // a shorter chunk of a pipelined launch (uniform)
     if (Q == 1 || (Q == 3 && J.W.kind == KIND_Q4K)) kq_tile<KIND_Q4K, NT, W, KS, NBH, PAIR>(J, UP, nb, row0, t0, S);
     else kq_tile<KIND_Q6K, NT, W, KS, NBH, PAIR>(J, UP, nb, row0, t0, S);
@@ -490,15 +466,7 @@ __global__ __launch_bounds__(64 * W * KS) void k_gemm_kq(GemmLaunchT<NJ> L) {
 
 template <int Q, int NJ, int NT, int W, int KS, int NBH, bool PAIR>
 hipError_t kq_go(GemmLaunchT<NJ>& L, hipStream_t s) {
-    int tiles = 0;
-    for (int q = 0; q < L.njobs; q++) {
-        if (PAIR && q % 2) {
-            L.job[q].tile_begin = 1 << 30;  // an up job: never selected by tile index
-            continue;
-        }
-        L.job[q].tile_begin = tiles;
-        tiles += (L.job[q].W.n + 16 * W - 1) / (16 * W);
-    }
+    const int tiles = gemm_tiles(L, 16 * W);
     k_gemm_kq<Q, NJ, NT, W, KS, NBH, PAIR><<<dim3(tiles, (L.nt + 16 * NT - 1) / (16 * NT)), 64 * W * KS, 0, s>>>(L);
     return hipGetLastError();
 }
