@@ -476,11 +476,14 @@ static bool run_mv1(Ctx* c, const JobSpec* js, int njobs, bool pair, const MvOpt
 // panels with the others, the general matvec kernel runs over groups of at most HY_MAX_BATCH
 // tokens. All give every token the single-token result. The threshold as measured on panels (a fused_forward of the config-3 model, matvec
 // against GEMM: 16 tokens 3.27 -> 1.95-2.01 ms, 8 tokens 2.34 -> 1.91-1.97, 4 tokens equal,
-// 2 tokens 1.71-1.78 against 1.87-1.92 ms)
+// 2 tokens 1.71-1.78 against 1.87-1.92 ms). Q4_K / Q6_K one token earlier (16 layers of a Q4_K_M
+// model: 2 tokens 965 against 1010 us, 3 tokens 1037 against 1019, 4 tokens 1110 against 1031; one
+// layer's contractions alone: 37.1 and 43.0, 42.3 and 43.7, 47.5 and 44.1).
 constexpr int kGemmMinTokens = 4;
+constexpr int kGemmKqMinTokens = 3;
 
 static bool run_multi(Ctx* c, const JobSpec* js, int njobs, bool pair, int nt, const MvOpts& o) {
-    if (nt > kGemmMinTokens && o.pro == PRO_NONE) {
+    if (nt > (js[0].w->mw.kind == KIND_PANEL ? kGemmMinTokens : kGemmKqMinTokens) && o.pro == PRO_NONE) {
         GemmLaunch G;
         memset(&G, 0, sizeof G);
         G.njobs = njobs;

@@ -894,6 +894,172 @@ __device__ __forceinline__ void attn_chunk_row(const AttnArgs& a, int g, int t) 
     }
 }
 
+// The same for launches of short rows (up to kAsPasses x 64 x 8 / GRP positions: 256 with four
+// heads a group), where one workgroup's phases, not the chip's work, take the time: a 16-token
+// batch is 64 workgroups. The group's heads go to different wavefronts, so that rows of a few dozen
+// positions occupy all of them: wavefront w scores head w % GRP for 64 keys a pass (k_attn_chunk
+// gives a key's every head to one lane: at 64 positions one wavefront then forms all scores), the
+// scores stay in registers until their exponentials, V tiles are double-buffered (the first one
+// stored before the scores' barrier), and a lane carries one output chain (8 wavefronts at head dim
+// 128, GRP 4). 16 tokens at positions 48-63: 13.7 -> 11.1 us a launch. A 32-layer forward, this form
+// against k_attn_chunk: 16 tokens at 0, 48, 112, 200: 1825, 1856, 1905, 2046 against 1949, 1940,
+// 2003, 2071 us; 64 tokens at 0: 2088 against 2153; 128 tokens at 0 and 100 (512 workgroups, several
+// a CU, whose throughput counts): 2573 and 2815 against 2561 and 2679, hence the workgroup limit.
+constexpr int kAsMaxWgs = 256;
+constexpr int kAsPasses = 2;
+constexpr int kAsTile = 64;  // positions per fp32 V tile
+
+template <int HD, int GRP>
+struct AsRow {
+    static constexpr int SH = kAcThreads / 64 / GRP;     // wavefronts per head in the scores
+    static constexpr int MAXN = kAsPasses * 64 * SH;     // positions a launch may reach
+};
+
+template <int HD, int GRP>
+__global__ __launch_bounds__(kAcThreads) void k_attn_chunk_short(AttnArgs a) {
+    constexpr int NW = kAcThreads / 64, KV4 = HD / 8, DW = HD / 64, SH = AsRow<HD, GRP>::SH, MAXN = AsRow<HD, GRP>::MAXN;
+    constexpr int VPT = kAsTile * KV4 / kAcThreads;  // 16-byte V pieces of a tile per thread
+    static_assert(NW % GRP == 0 && GRP * DW <= NW && kAsTile * KV4 % kAcThreads == 0, "heads over the wavefronts");
+    __shared__ __align__(16) float sc[GRP][MAXN];            // e_j, then p_j
+    __shared__ __align__(16) float vt[2][kAsTile * HD];      // fp32 V tiles [j][d]
+    __shared__ float red[GRP][SH];
+    __shared__ float inv_s[GRP];
+    __shared__ uint64_t etab[32];
+    // the arguments in one round of scalar loads
+    asm volatile("" ::"s"(a.q), "s"(a.kc), "s"(a.vc), "s"(a.ao), "s"(a.pos0), "s"(a.heads), "s"(a.ctx), "s"(a.act_out));
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = blockIdx.x, t = blockIdx.y, pos = a.pos0 + t, n = pos + 1, qdim = a.heads * HD;
+    const uint16_t* K = a.kc + (size_t)g * a.ctx * HD;
+    const uint16_t* V = a.vc + (size_t)g * a.ctx * HD;
+    const int hh = wave % GRP, kw = wave / GRP;
+
+    v4u kr[KV4], vr[VPT];
+    auto load_key = [&](int j) __attribute__((always_inline)) {
+        const uint16_t* row = K + (size_t)min(j, pos) * HD;
+#pragma unroll
+        for (int i = 0; i < KV4; i++) kr[i] = *reinterpret_cast<const v4u*>(row + 8 * i);
+    };
+    auto load_v = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < VPT; i++) {
+            const int f = tid + kAcThreads * i;
+            vr[i] = *reinterpret_cast<const v4u*>(V + (size_t)min(t0 + f / KV4, pos) * HD + 8 * (f % KV4));
+        }
+    };
+    auto store_v = [&](float* tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < VPT; i++) {
+            const int f = tid + kAcThreads * i;
+            float* d = tile + (f / KV4) * HD + 8 * (f % KV4);
+            const v4u w = vr[i];
+            *reinterpret_cast<float4*>(d) =
+                make_float4(hy_bitsf(w.x << 16), hy_bitsf(w.x & 0xffff0000u), hy_bitsf(w.y << 16), hy_bitsf(w.y & 0xffff0000u));
+            *reinterpret_cast<float4*>(d + 4) =
+                make_float4(hy_bitsf(w.z << 16), hy_bitsf(w.z & 0xffff0000u), hy_bitsf(w.w << 16), hy_bitsf(w.w & 0xffff0000u));
+        }
+    };
+    load_key(64 * kw + lane);
+    load_v(0);
+    if (tid < 32) etab[tid] = hy_exp_tab_entry(tid);  // read after the barrier past the scores
+
+    // scores of this wavefront's head, key 64 (kw + SH p) + lane in pass p; q through the constant
+    // address space (scalar loads, as in attn_chunk_row)
+    typedef __attribute__((address_space(4))) const float cfloat;
+    const uint64_t qaddr = (uint64_t)(uintptr_t)(a.q + (size_t)t * qdim + (size_t)(g * GRP + hh) * HD);
+    const float scale = 1.0f / sqrtf((float)HD);
+    float s[kAsPasses], lm = -__builtin_inff();
+#pragma unroll
+    for (int p = 0; p < kAsPasses; p++) {
+        const int j0 = 64 * (kw + SH * p);
+        if (j0 >= n) break;
+        if (p) load_key(j0 + lane);
+        const cfloat* qh = (const cfloat*)qaddr;
+        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < KV4; i++) {
+            const v4u kv = kr[i];
+            const float kf[8] = {hy_bitsf(kv.x << 16), hy_bitsf(kv.x & 0xffff0000u), hy_bitsf(kv.y << 16),
+                                 hy_bitsf(kv.y & 0xffff0000u), hy_bitsf(kv.z << 16), hy_bitsf(kv.z & 0xffff0000u),
+                                 hy_bitsf(kv.w << 16), hy_bitsf(kv.w & 0xffff0000u)};
+#pragma unroll
+            for (int c = 0; c < 8; c++) acc[c & 3] += qh[8 * i + c] * kf[c];
+        }
+        s[p] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) * scale;
+        if (j0 + lane < n) lm = fmaxf(lm, s[p]);
+    }
+    lm = hy_wave_max(lm);
+    if (lane == 0) red[hh][kw] = lm;
+    store_v(vt[0]);
+    if (kAsTile < n) load_v(kAsTile);
+    __syncthreads();
+    float mx = red[hh][0];
+#pragma unroll
+    for (int w = 1; w < SH; w++) mx = fmaxf(mx, red[hh][w]);
+#pragma unroll
+    for (int p = 0; p < kAsPasses; p++) {
+        const int j = 64 * (kw + SH * p) + lane;
+        if (j - lane >= n) break;
+        if (j < n) sc[hh][j] = hy_expf_tab(s[p] - mx, etab);
+    }
+    __syncthreads();
+    // the heads' sums in position order, together in the 16-lane rows of wavefront 0
+    if (wave == 0) {
+        float sum[4];
+        hy_row_seq_sums<GRP>(&sc[0][0], MAXN, n, lane, sum);
+        if (lane == 0)
+#pragma unroll
+            for (int h = 0; h < GRP; h++) inv_s[h] = 1.0f / sum[h];
+    }
+    __syncthreads();
+    // p_j = e_j * inv, once per position, by the wavefronts that formed e_j
+    const float inv = inv_s[hh];
+#pragma unroll
+    for (int p = 0; p < kAsPasses; p++) {
+        const int j = 64 * (kw + SH * p) + lane;
+        if (j < n) sc[hh][j] = sc[hh][j] * inv;
+    }
+    __syncthreads();
+    // output chains, one head (oh) and dimension (od) a lane
+    const int oh = wave / DW, od = (wave % DW) * 64 + lane;
+    float o = 0.f;
+    for (int t0 = 0, b = 0; t0 < n; t0 += kAsTile, b ^= 1) {
+        if (t0) __syncthreads();  // this tile stored, the one before it (the other buffer) read
+        if (t0 + kAsTile < n) {
+            store_v(vt[b ^ 1]);
+            if (t0 + 2 * kAsTile < n) load_v(t0 + 2 * kAsTile);
+        }
+        if (oh < GRP) {
+            const float* vd = vt[b] + od;
+            const float* pj = sc[oh] + t0;
+            const int cnt = min(kAsTile, n - t0);
+            int q = 0;
+            for (; q + 16 <= cnt; q += 16) {
+                float vv[16], pv[16];
+#pragma unroll
+                for (int k = 0; k < 16; k++) vv[k] = vd[(q + k) * HD];
+#pragma unroll
+                for (int k = 0; k < 16; k += 4) {
+                    const float4 x = *reinterpret_cast<const float4*>(pj + q + k);
+                    pv[k] = x.x, pv[k + 1] = x.y, pv[k + 2] = x.z, pv[k + 3] = x.w;
+                }
+#pragma unroll
+                for (int k = 0; k < 16; k++) o += pv[k] * vv[k];
+            }
+            for (; q < cnt; q++) o += pj[q] * vd[q * HD];
+        }
+    }
+    if (oh < GRP) a.ao[(size_t)t * qdim + (size_t)(g * GRP + oh) * HD + od] = o;
+    if constexpr (GRP * HD % HY_QK == 0) {
+        if (a.act_out) {
+            constexpr int NB = GRP * HD / HY_QK;
+            __syncthreads();  // every chain has read its last tile
+            if (oh < GRP) vt[0][oh * HD + od] = o;
+            __syncthreads();
+            if (wave < NB) q8k_quantize_wave(vt[0] + wave * HY_QK, a.act_out + (size_t)t * (qdim / HY_QK) + g * NB + wave, lane);
+        }
+    }
+}
+
 template <int HD, int GRP>
 __global__ __launch_bounds__(kAcThreads) void k_attn_chunk(AttnArgs a) {
     attn_chunk_row<HD, GRP, kAcTileRow>(a, blockIdx.x, blockIdx.y);
@@ -1258,6 +1424,17 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t s) {
         J.njobs = 1;
         hipError_t e;
         if (launch_attn4(J, s, e)) return e;
+    }
+    if (a.ctx <= kAcMaxCtx && !a.pos_dev && a.kv_heads * a.nt <= kAsMaxWgs) {
+        const dim3 grid(a.kv_heads, a.nt);
+        const int last = a.pos0 + a.nt;
+        if (a.hdim == 128 && grp == 4 && last <= AsRow<128, 4>::MAXN) k_attn_chunk_short<128, 4><<<grid, kAcThreads, 0, s>>>(a);
+        else if (a.hdim == 128 && grp == 2 && last <= AsRow<128, 2>::MAXN) k_attn_chunk_short<128, 2><<<grid, kAcThreads, 0, s>>>(a);
+        else if (a.hdim == 64 && grp == 4 && last <= AsRow<64, 4>::MAXN) k_attn_chunk_short<64, 4><<<grid, kAcThreads, 0, s>>>(a);
+        else if (a.hdim == 64 && grp == 2 && last <= AsRow<64, 2>::MAXN) k_attn_chunk_short<64, 2><<<grid, kAcThreads, 0, s>>>(a);
+        else grp = 0;
+        if (grp) return hipGetLastError();
+        grp = a.heads % a.kv_heads == 0 ? a.heads / a.kv_heads : 0;
     }
     if (a.ctx <= kAcMaxCtx) {
         const dim3 grid(a.kv_heads, a.nt);
