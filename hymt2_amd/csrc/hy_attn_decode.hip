@@ -1,6 +1,6 @@
-// Single-token attention of the fused decode step (nt = 1), gfx950: one 512-thread workgroup
-// per query head, the reference's attn_task for one position (src/model.c:767-795) after the
-// per-token RoPE, q/k RMSNorm and bf16 KV store (src/model.c:836-847).
+// Single-token attention of the fused decode step (nt = 1), gfx950: one or two 512-thread workgroups
+// per query head (a1_parts, each its own output dimensions), the reference's attn_task for one position
+// (src/model.c:767-795) after the per-token RoPE, q/k RMSNorm and bf16 KV store (src/model.c:836-847).
 //
 // Scores: one key per thread per pass of 512 positions, dot_bf16's four interleaved partial
 // sums in order (src/kernels.c:1111-1121); the first pass's key rows load at kernel entry. Softmax
@@ -8,8 +8,8 @@
 // exact segmented sum (hy_block_exact_sum8), p_j = e_j * (1 / sum) formed once per position.
 // Output (axpy_bf16, src/kernels.c:1122-1124): o[d] += p_j * V_j[d] in position order, as a
 // pipeline over tiles of 96 positions: wavefronts 2-7 convert the V rows of tile t + 1 to fp32
-// into one half of a double-buffered [j][d] LDS tile while wavefronts 0-1 (one lane per
-// dimension) walk tile t in position order, each step one multiply p_j * V_j[d] (rounded to fp32,
+// into one half of a double-buffered [j][d] LDS tile while wavefront 0 (head dim 128: the
+// workgroup's 64 dimensions, one a lane) walks tile t in position order, each step one multiply p_j * V_j[d] (rounded to fp32,
 // as the reference rounds it) and one add; one LDS-only barrier per tile, V rows loaded three
 // tiles ahead. The fp32 output row goes to `ao`; the o-projection quantizes it.
 #include "hy_kernels.h"
@@ -17,6 +17,15 @@
 namespace hy {
 
 namespace {
+
+// Workgroups per query head, each with its own run of output dimensions; the scores and the softmax are
+// every one's. A workgroup's K and V rows pass through one CU at about 48 bytes a ns, so halving its V
+// (and the fp32 stage, whose LDS then holds short rows of 256 positions instead of 192) shortens every
+// row: decode of the 32-layer ternary model at positions 64-128, 110-158, 180-240, 260-320, 370-430:
+// 856, 880, 951, 1028, 1102 us a token with one workgroup, 851, 867, 911, 983, 1033 with two (four:
+// 852, 871, 912, 979, 1035).
+template <int HD>
+constexpr int a1_parts() { return HD == 128 ? 2 : 1; }
 
 constexpr int kA1Threads = 512;
 constexpr int kA1Waves = kA1Threads / 64;
@@ -26,7 +35,7 @@ constexpr int kA1Chunk = 32;           // positions per chain step (16 LDS reads
 constexpr int kA1SerialSum = 256;      // softmax rows up to this length: the lane-serial sum
 constexpr int kA1PairRow = kA1Threads / 2;  // rows up to this length: two lanes per key
 static_assert(kA1SerialSum <= kA1PairRow, "the serial sum reads the pair form's padded exponentials");
-constexpr int kA1ShortRow = 2 * kA1Tile;    // rows up to this length: V staged whole, direct chains
+constexpr int kA1ShortRow = kA1PairRow;     // rows up to this length: V staged whole, direct chains
 
 __device__ __forceinline__ void bf16x8f(const uint4& v, float* f) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -148,18 +157,18 @@ __device__ __forceinline__ void a1_load_key(uint4 (&k)[HD / 8], const uint16_t* 
 // (0 .. kA1Prod - 1) owns quad p % QPR of rows p / QPR + RSTEP k, k < IPT, of every tile: a
 // wavefront's loads of one k cover whole rows (contiguous global memory), its product stores
 // one contiguous run of the [j][d] tile.
-template <int HD>
+template <int VD>
 struct A1Split {
-    static constexpr int QPR = HD / 4;                   // quads per row
+    static constexpr int QPR = VD / 4;                   // quads per row
     static constexpr int IPT = kA1Tile * QPR / kA1Prod;  // quads per producer thread per tile
     static constexpr int RSTEP = kA1Prod / QPR;          // rows between a thread's quads
     static_assert(kA1Prod % QPR == 0 && kA1Tile % RSTEP == 0, "whole rows per producer step");
 };
 
 // V quads of one tile for producer thread p: rows t0 + row (clamped to `last`)
-template <int HD>
-__device__ __forceinline__ void a1_load_v(uint2 (&v)[A1Split<HD>::IPT], const uint16_t* V, int t0, int p, int last) {
-    using P = A1Split<HD>;
+template <int HD, int VD>
+__device__ __forceinline__ void a1_load_v(uint2 (&v)[A1Split<VD>::IPT], const uint16_t* V, int t0, int p, int last) {
+    using P = A1Split<VD>;
     const int r0 = t0 + p / P::QPR, q = p % P::QPR;
 #pragma unroll
     for (int k = 0; k < P::IPT; k++)
@@ -173,7 +182,7 @@ __device__ __forceinline__ void a1_load_v(uint2 (&v)[A1Split<HD>::IPT], const ui
 // cancels rounds to +0). The reads of the next chunk are issued before a chunk is added, and
 // scheduling barriers keep them there: left to itself the compiler moves each read next to its
 // use, and the chain then waits out the LDS latency at every position.
-template <int HD>
+template <int VD>
 __device__ __forceinline__ void a1_chain(const float* col, const float* pj, int nch, float& o) {
     static_assert(kA1Tile == 3 * kA1Chunk, "three chunks per tile");
     constexpr int C = kA1Chunk / 2;  // positions per step
@@ -185,7 +194,7 @@ __device__ __forceinline__ void a1_chain(const float* col, const float* pj, int 
             p[i] = q.x, p[i + 1] = q.y, p[i + 2] = q.z, p[i + 3] = q.w;
         }
 #pragma unroll
-        for (int i = 0; i < C; i++) v[i] = col[(j0 + i) * HD];
+        for (int i = 0; i < C; i++) v[i] = col[(j0 + i) * VD];
     };
     auto add = [&](const float (&v)[C], const float (&p)[C]) __attribute__((always_inline)) {
 #pragma unroll
@@ -208,10 +217,10 @@ __device__ __forceinline__ void a1_chain(const float* col, const float* pj, int 
 // V rows of one tile as fp32 into buf[j][d] (16-byte stores) for producer thread p's quads.
 // EDGE (the tile reaches the row's end): position `pos` takes this token's V row from LDS (vb,
 // all read before any value is stored) and positions past the row are +0.
-template <int HD, bool EDGE>
-__device__ __forceinline__ void a1_stage_tile(const uint2 (&v)[A1Split<HD>::IPT], float* buf, const uint16_t* vb,
+template <int VD, bool EDGE>
+__device__ __forceinline__ void a1_stage_tile(const uint2 (&v)[A1Split<VD>::IPT], float* buf, const uint16_t* vb,
                                               int t0, int p, int pos, int n) {
-    using P = A1Split<HD>;
+    using P = A1Split<VD>;
     const int r0 = p / P::QPR, q = p % P::QPR;
     uint2 w[P::IPT];
 #pragma unroll
@@ -230,16 +239,16 @@ __device__ __forceinline__ void a1_stage_tile(const uint2 (&v)[A1Split<HD>::IPT]
         float4 x = make_float4(hy_bitsf(w[k].x << 16), hy_bitsf(w[k].x & 0xffff0000u), hy_bitsf(w[k].y << 16),
                                hy_bitsf(w[k].y & 0xffff0000u));
         if (EDGE && t0 + r >= n) x = {0.f, 0.f, 0.f, 0.f};
-        *reinterpret_cast<float4*>(buf + r * HD + 4 * q) = x;
+        *reinterpret_cast<float4*>(buf + r * VD + 4 * q) = x;
     }
 }
 
 // Short rows: V of the tile at t0 as fp32 into stage[j][d] for producer thread p's quads (rows
 // below n; position `pos` from this token's V row in LDS, vb).
-template <int HD>
-__device__ __forceinline__ void a1_stage_v(const uint2 (&v)[A1Split<HD>::IPT], float* stage, const uint16_t* vb,
+template <int VD>
+__device__ __forceinline__ void a1_stage_v(const uint2 (&v)[A1Split<VD>::IPT], float* stage, const uint16_t* vb,
                                            int t0, int p, int pos, int n) {
-    using P = A1Split<HD>;
+    using P = A1Split<VD>;
     const int r0 = t0 + p / P::QPR, q = p % P::QPR;
     const uint2 b = *reinterpret_cast<const uint2*>(vb + 4 * q);
 #pragma unroll
@@ -247,7 +256,7 @@ __device__ __forceinline__ void a1_stage_v(const uint2 (&v)[A1Split<HD>::IPT], f
         const int r = r0 + P::RSTEP * k;
         if (r < n) {
             const uint2 w = r == pos ? b : v[k];
-            *reinterpret_cast<float4*>(stage + r * HD + 4 * q) =
+            *reinterpret_cast<float4*>(stage + r * VD + 4 * q) =
                 make_float4(hy_bitsf(w.x << 16), hy_bitsf(w.x & 0xffff0000u), hy_bitsf(w.y << 16), hy_bitsf(w.y & 0xffff0000u));
         }
     }
@@ -258,7 +267,7 @@ __device__ __forceinline__ void a1_stage_v(const uint2 (&v)[A1Split<HD>::IPT], f
 // while a chunk is added (a loop over chunk pairs, so that no exit sits between a prefetch and
 // its use for the compiler to sink the prefetch behind); each step is one multiply independent
 // of the chain and one add on it. Reads stay inside the stage (positions < kA1ShortRow).
-template <int HD>
+template <int VD>
 __device__ __forceinline__ float a1_short_chain(const float* col, const float* pj, int n) {
     constexpr int C = 16, LIM = kA1ShortRow - C;
     float ea[C], va[C], eb[C], vb[C];
@@ -269,7 +278,7 @@ __device__ __forceinline__ float a1_short_chain(const float* col, const float* p
             e[i] = q.x, e[i + 1] = q.y, e[i + 2] = q.z, e[i + 3] = q.w;
         }
 #pragma unroll
-        for (int i = 0; i < C; i++) v[i] = col[(j0 + i) * HD];
+        for (int i = 0; i < C; i++) v[i] = col[(j0 + i) * VD];
     };
     float o = 0.f;
     auto add = [&](const float (&e)[C], const float (&v)[C]) __attribute__((always_inline)) {
@@ -316,34 +325,39 @@ __device__ __forceinline__ float a1_short_chain(const float* col, const float* p
 // rows three tiles on. The loads are unconditional so that every path through a group of three
 // steps leaves the same loads in flight, and the compiler's wait before a tile's stores leaves
 // the later tiles' loads outstanding.
-template <int HD>
-__device__ __forceinline__ void a1_produce(uint2 (&v)[A1Split<HD>::IPT], float* buf, const uint16_t* vb,
+template <int HD, int VD>
+__device__ __forceinline__ void a1_produce(uint2 (&v)[A1Split<VD>::IPT], float* buf, const uint16_t* vb,
                                            const uint16_t* V, int t0, int p, int pos, int n, int last) {
     if (t0 < n) {
-        if (t0 + kA1Tile < n) a1_stage_tile<HD, false>(v, buf, vb, t0, p, pos, n);
-        else a1_stage_tile<HD, true>(v, buf, vb, t0, p, pos, n);
+        if (t0 + kA1Tile < n) a1_stage_tile<VD, false>(v, buf, vb, t0, p, pos, n);
+        else a1_stage_tile<VD, true>(v, buf, vb, t0, p, pos, n);
     }
-    a1_load_v<HD>(v, V, t0 + 3 * kA1Tile, p, last);
+    a1_load_v<HD, VD>(v, V, t0 + 3 * kA1Tile, p, last);
     if (t0 < n) hy_lds_barrier();
 }
 
-// The query head of this k_attn1 workgroup. Workgroups go to the 8 XCDs round-robin (workgroup b
-// on XCD b % 8), each XCD with its own L2: consecutive heads share an XCD (heads 2x, 2x + 1 on XCD
-// x for 16 heads), so a KV head's K and V rows are fetched by half as many L2s as in id order
-// (measured 5.5x the algorithmic bytes in id order at 4 query heads per KV head). Head counts
-// that are not a multiple of 8 keep id order.
-__device__ __forceinline__ int a1_head(int heads) {
-    const int b = blockIdx.x;
-    return heads % 8 ? b : (b % 8) * (heads / 8) + b / 8;
+// The query head of this k_attn1 workgroup and which of the head's PARTS runs of output dimensions it
+// takes. Workgroups go to the 8 XCDs round-robin (workgroup b on XCD b % 8), each XCD with its own
+// L2: consecutive heads share an XCD (heads 2x, 2x + 1 on XCD x for 16 heads), so a KV head's K and V
+// rows are fetched by half as many L2s as in id order (measured 5.5x the algorithmic bytes in id order
+// at 4 query heads per KV head). Counts that are not a multiple of 8 keep id order.
+template <int PARTS>
+__device__ __forceinline__ int a1_head(int heads, int& part) {
+    const int b = blockIdx.x, n = heads * PARTS;
+    const int u = n % 8 ? b : (b % 8) * (n / 8) + b / 8;
+    part = u % PARTS;
+    return u / PARTS;
 }
 
 // LDS of one head's attention.
 template <int HD>
 struct A1Smem {
+    static constexpr int VD = HD / a1_parts<HD>();
     alignas(16) float ex[(kA1MaxCtx + kA1Tile - 1) / kA1Tile * kA1Tile];  // e_j = expf(s_j - max), then p_j
     union {
         HyExactLdsT<kA1Waves> exs;            // the softmax sum of long rows
-        alignas(16) float prod[2][kA1Tile * HD];  // then the products of two tiles, [j][d]
+        alignas(16) float prod[2][kA1Tile * VD];  // then V of two tiles, [j][d]
+        alignas(16) float stage[kA1ShortRow * VD];  // short rows: V whole
     };
     alignas(16) float scr[2][HD];
     alignas(16) float qn[HD];
@@ -358,11 +372,12 @@ struct A1Smem {
 // q / k / v elements lane + 64 i for wavefronts 0 / 1 / 2), its RoPE row (rc, rs) and the q / k
 // norm weights (nw) are loaded; the key rows of the first pass (kA, rows below pos) and, in the
 // producer wavefronts (2-7), the first V tile (v0) are in flight.
-template <int HD>
+template <int HD, int VD = A1Smem<HD>::VD>
 __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const float (&x)[HD / 64],
                                         const float (&rc)[HD / 64], const float (&rs)[HD / 64],
-                                        const float (&nw)[HD / 64], uint4 (&kA)[HD / 8], uint2 (&v0)[A1Split<HD>::IPT],
-                                        uint2 (&v1)[A1Split<HD>::IPT], int pos, uint64_t etv) {
+                                        const float (&nw)[HD / 64], uint4 (&kA)[HD / 8], uint2 (&v0)[A1Split<VD>::IPT],
+                                        uint2 (&v1)[A1Split<VD>::IPT], uint2 (&v2)[A1Split<VD>::IPT],
+                                        int pos, uint64_t etv) {
     constexpr int KV4 = HD / 8;                 // 16-byte pieces of one K / V row
     constexpr int RPL = HD / 64;                // row elements per lane
     constexpr int PASSES = kA1MaxCtx / kA1Threads;
@@ -371,22 +386,22 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
     float(&scr)[2][HD] = S.scr;
     float* qn = S.qn;
     uint16_t* kb = S.kb;
-    uint16_t* vb = S.vb;
     float* red = S.red;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = a1_head(a.heads);
+    int part;  // this workgroup's output dimensions: VD from part * VD
+    const int h = a1_head<HD / VD>(a.heads, part);
+    uint16_t* vb = S.vb + part * VD;  // this token's V row at them
     const int group = a.heads / a.kv_heads;
     const int g = h / group;
     const int half = a.rope_half;
     const int cap = a.ctx - 1;
     const uint16_t* K = a.kc + (size_t)g * a.ctx * HD;
-    const uint16_t* V = a.vc + (size_t)g * a.ctx * HD;
+    const uint16_t* V = a.vc + (size_t)g * a.ctx * HD + part * VD;
     const bool prd = wave >= 2;
     const int pp = prd ? tid - 128 : lane;  // producer index (other wavefronts: any valid one)
     const int n = pos + 1;
     uint4 kB[KV4];
-    uint2 v2[A1Split<HD>::IPT];
 
     // 1. RoPE + RMSNorm of q (wavefront 0) and k (1), bf16 of k and v
     if (wave < 2) {
@@ -399,15 +414,15 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
         }
     } else if (wave == 2) {
 #pragma unroll
-        for (int i = 0; i < RPL; i++) vb[lane + 64 * i] = hy_to_bf16(x[i]);
+        for (int i = 0; i < RPL; i++) S.vb[lane + 64 * i] = hy_to_bf16(x[i]);
     }
     // LDS only: a full __syncthreads would also wait for every key and V row in flight
     hy_lds_barrier();
     // the bf16 k, v of this position (src/model.c:842-847), stored once per KV head
-    if (h % group == 0 && tid < HD) {
+    if (h % group == 0 && part == 0 && tid < HD) {
         const size_t off = ((size_t)g * a.ctx + pos) * HD + tid;
         a.kc[off] = kb[tid];
-        a.vc[off] = vb[tid];
+        a.vc[off] = S.vb[tid];
     }
 
     // 2. scores s_j = dot_bf16(q, K_j) * (1/sqrtf(hd)) for j = tid + 512 p, kept in registers;
@@ -448,8 +463,8 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
     // producers' waits leave them out (short rows loaded tile 1 at entry).
     const int last = max(pos - 1, 0);
     if (prd && n > kA1ShortRow) {
-        a1_load_v<HD>(v1, V, kA1Tile, pp, last);
-        a1_load_v<HD>(v2, V, 2 * kA1Tile, pp, last);
+        a1_load_v<HD, VD>(v1, V, kA1Tile, pp, last);
+        a1_load_v<HD, VD>(v2, V, 2 * kA1Tile, pp, last);
     }
     a1_fence();  // issued here, not next to their first use
     lmax = hy_wave_max(lmax);
@@ -488,8 +503,9 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
                     for (int j = lane; j < n; j += 64) ex[j] = ex[j] * iv;
                 }
             } else if (n <= kA1ShortRow && prd) {  // meanwhile the producers stage V whole
-                a1_stage_v<HD>(v0, &S.prod[0][0], vb, 0, pp, pos, n);
-                if (n > kA1Tile) a1_stage_v<HD>(v1, &S.prod[0][0], vb, kA1Tile, pp, pos, n);
+                a1_stage_v<VD>(v0, S.stage, vb, 0, pp, pos, n);
+                if (n > kA1Tile) a1_stage_v<VD>(v1, S.stage, vb, kA1Tile, pp, pos, n);
+                if (n > 2 * kA1Tile) a1_stage_v<VD>(v2, S.stage, vb, 2 * kA1Tile, pp, pos, n);
             }
             hy_lds_barrier();
             inv = S.stat;
@@ -521,26 +537,26 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
     //    ahead, in groups of three steps (one loop exit; steps past the row only load).
     // Short rows: every lane of wavefronts 0 .. HD/64 - 1 walks its dimension over the staged V.
     if (n <= kA1ShortRow) {
-        static_assert(kA1ShortRow <= kA1SerialSum && kA1ShortRow * HD <= 2 * kA1Tile * HD, "staged V fits");
-        if (wave < HD / 64) a.ao[(size_t)h * HD + tid] = a1_short_chain<HD>(&S.prod[0][0] + tid, ex, n);
+        static_assert(kA1ShortRow <= kA1SerialSum && kA1ShortRow <= 3 * kA1Tile, "three tiles of V, one sum");
+        if (tid < VD) a.ao[(size_t)h * HD + part * VD + tid] = a1_short_chain<VD>(S.stage + tid, ex, n);
         return;
     }
     const int tiles = (n + kA1Tile - 1) / kA1Tile;
-    if (wave < HD / 64) {
+    if (wave < (VD + 63) / 64) {
         __builtin_amdgcn_s_setprio(3);  // the chain is the critical path: its adds issue first
         float o = 0.f;
         for (int t = 0; t < tiles; t++) {
             hy_lds_barrier();
             const int cnt = min(kA1Tile, n - t * kA1Tile);
-            a1_chain<HD>(S.prod[t & 1] + tid, ex + t * kA1Tile, (cnt + kA1Chunk - 1) / kA1Chunk, o);
+            a1_chain<VD>(S.prod[t & 1] + tid % VD, ex + t * kA1Tile, (cnt + kA1Chunk - 1) / kA1Chunk, o);
         }
-        a.ao[(size_t)h * HD + tid] = o;
+        if (tid < VD) a.ao[(size_t)h * HD + part * VD + tid] = o;
     } else if (prd) {
         for (int t = 0; t < tiles; t += 3) {
             const int t0 = t * kA1Tile;
-            a1_produce<HD>(v0, S.prod[t & 1], vb, V, t0, pp, pos, n, last);
-            a1_produce<HD>(v1, S.prod[(t + 1) & 1], vb, V, t0 + kA1Tile, pp, pos, n, last);
-            a1_produce<HD>(v2, S.prod[t & 1], vb, V, t0 + 2 * kA1Tile, pp, pos, n, last);
+            a1_produce<HD, VD>(v0, S.prod[t & 1], vb, V, t0, pp, pos, n, last);
+            a1_produce<HD, VD>(v1, S.prod[(t + 1) & 1], vb, V, t0 + kA1Tile, pp, pos, n, last);
+            a1_produce<HD, VD>(v2, S.prod[t & 1], vb, V, t0 + 2 * kA1Tile, pp, pos, n, last);
         }
     } else {
         for (int t = 0; t < tiles; t++) hy_lds_barrier();
@@ -549,7 +565,7 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
 
 template <int HD>
 __global__ __launch_bounds__(kA1Threads) void k_attn1(Attn1Args a) {
-    constexpr int RPL = HD / 64;
+    constexpr int RPL = HD / 64, VD = A1Smem<HD>::VD;
     __shared__ A1Smem<HD> S;
     // Every kernel argument in one round of scalar loads, pinned in SGPRs before use: the
     // per-wavefront selections below would otherwise chain dependent loads of the arguments.
@@ -558,11 +574,12 @@ __global__ __launch_bounds__(kA1Threads) void k_attn1(Attn1Args a) {
         hy_sgpr_pin(a.pos_dev), hy_sgpr_pin(a.rope_cur), hy_sgpr_pin(a.pos0), hy_sgpr_pin(a.ao), hy_sgpr_pin(a.heads),
         hy_sgpr_pin(a.kv_heads), hy_sgpr_pin(a.rope_half), hy_sgpr_pin(a.ctx), hy_sgpr_pin(a.eps);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = a1_head(a.heads);
+    int part;
+    const int h = a1_head<HD / VD>(a.heads, part);
     const int g = h / (a.heads / a.kv_heads);
     const int half = a.rope_half;
     const uint16_t* K = a.kc + (size_t)g * a.ctx * HD;
-    const uint16_t* V = a.vc + (size_t)g * a.ctx * HD;
+    const uint16_t* V = a.vc + (size_t)g * a.ctx * HD + part * VD;
     const bool prd = wave >= 2;
     const int pp = prd ? tid - 128 : lane;
 
@@ -606,19 +623,20 @@ __global__ __launch_bounds__(kA1Threads) void k_attn1(Attn1Args a) {
     } else if (tid < pos) {
         a1_load_key<HD>(kA, K, tid);
     }
-    uint2 v0[A1Split<HD>::IPT], v1[A1Split<HD>::IPT];
-    a1_load_v<HD>(v0, V, 0, pp, max(pos - 1, 0));
-    // short rows past one tile: the producers' second tile too, staged during the softmax sum
-    if (prd && pos >= kA1Tile && pos < kA1ShortRow) a1_load_v<HD>(v1, V, kA1Tile, pp, pos - 1);
+    uint2 v0[A1Split<VD>::IPT], v1[A1Split<VD>::IPT], v2[A1Split<VD>::IPT];
+    a1_load_v<HD, VD>(v0, V, 0, pp, max(pos - 1, 0));
+    // short rows past one tile: the producers' other tiles too, staged during the softmax sum
+    if (prd && pos >= kA1Tile && pos < kA1ShortRow) a1_load_v<HD, VD>(v1, V, kA1Tile, pp, pos - 1);
+    if (prd && pos >= 2 * kA1Tile && pos < kA1ShortRow) a1_load_v<HD, VD>(v2, V, 2 * kA1Tile, pp, pos - 1);
     a1_fence();
-    a1_core<HD>(a, S, x, rc, rs, nw, kA, v0, v1, pos, etv);
+    a1_core<HD>(a, S, x, rc, rs, nw, kA, v0, v1, v2, pos, etv);
 }
 
 hipError_t launch_attn1(const Attn1Args& a, hipStream_t s) {
     if (a.heads % a.kv_heads || 2 * a.rope_half > a.hdim || a.ctx > kA1MaxCtx) return hipErrorNotSupported;
     switch (a.hdim) {
-    case 64: k_attn1<64><<<a.heads, kA1Threads, 0, s>>>(a); break;
-    case 128: k_attn1<128><<<a.heads, kA1Threads, 0, s>>>(a); break;
+    case 64: k_attn1<64><<<a.heads * a1_parts<64>(), kA1Threads, 0, s>>>(a); break;
+    case 128: k_attn1<128><<<a.heads * a1_parts<128>(), kA1Threads, 0, s>>>(a); break;
     default: return hipErrorNotSupported;
     }
     return hipGetLastError();
