@@ -80,7 +80,12 @@ struct Fused {
     size_t in_bytes = 0;
     float *q = nullptr, *k = nullptr, *v = nullptr, *ao = nullptr, *g = nullptr, *u = nullptr, *logits = nullptr;
     HyQ8K *act_h = nullptr, *act_q = nullptr, *act_f = nullptr;
-    float *rope_c = nullptr, *rope_s = nullptr, *out_norm = nullptr, *norms = nullptr;
+    // the model's parameters besides its weights, in one device array (copy_params): the layers'
+    // norms, the output norm, the RoPE tables; and the same bytes as last uploaded
+    char* par = nullptr;
+    std::vector<char> par_host;
+    bool par_sent = false;
+    float *rope_c = nullptr, *rope_s = nullptr, *out_norm = nullptr, *norms = nullptr;  // in par
     uint16_t *kc = nullptr, *vc = nullptr;
     size_t logits_cap = 0;
     unsigned long long* slots = nullptr;  // argmax keys of the LM head, one per workgroup (kArgSlots)
@@ -673,7 +678,7 @@ static void free_fused(Fused* f) {
     if (!f) return;
     free_graphs(f);
     void* dev[] = {f->in_dev,  f->q,       f->k,       f->v,       f->ao,    f->g,       f->u,     f->logits,
-                   f->act_h,   f->act_q,   f->act_f,   f->rope_c,  f->rope_s, f->out_norm, f->norms, f->kc,
+                   f->act_h,   f->act_q,   f->act_f,   f->par,     f->kc,
                    f->vc,      f->slots,   f->ids,     f->sc,      f->segmax, f->p_h,     f->p_q,   f->p_k,
                    f->p_v,     f->p_ao,    f->p_g,     f->p_act_h, f->p_act_q, f->p_act_f};
     for (void* p : dev)
@@ -694,17 +699,43 @@ static bool same_shape(const Fused* f, const hymt2_fused_args* a) {
 // (reference cu_fused_prepare, src/cuda.c:282-337; idempotent for the same shape).
 static bool copy_params(Ctx* c, const hymt2_fused_args* a) {
     Fused* f = c->f;
-    const size_t H = f->hidden;
-    const size_t rb = (size_t)a->ctx * a->rope_half * 4;
-    HIPCHK(c, hipMemcpy(f->rope_c, a->rope_cos, rb, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(f->rope_s, a->rope_sin, rb, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(f->out_norm, a->out_norm, H * 4, hipMemcpyHostToDevice));
+    const size_t H = (size_t)f->hidden * 4, D = (size_t)f->hdim * 4, rb = (size_t)a->ctx * a->rope_half * 4;
+    // One upload of what differs from the last one (usually nothing: a device loop prepares again at
+    // every call). A copy for each array, 131 for 32 layers, each waited for, took about 1.3 ms a
+    // call, two calls a generate_ids.
+    bool ok = true, changed = !f->par_sent;
+    auto put = [&](const float* dev, const float* src, size_t bytes) {
+        if (!bytes) return;
+        if (!src) {
+            ok = false;
+            return;
+        }
+        char* h = f->par_host.data() + (reinterpret_cast<const char*>(dev) - f->par);
+        if (memcmp(h, src, bytes)) {
+            memcpy(h, src, bytes);
+            changed = true;
+        }
+    };
     for (int li = 0; li < a->n_layer; li++) {
         const hymt2_fused_layer& L = a->layers[li];
-        HIPCHK(c, hipMemcpy(f->norm_ptr(li, 0), L.attn_norm, H * 4, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(f->norm_ptr(li, 1), L.ffn_norm, H * 4, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(f->norm_ptr(li, 2), L.q_norm, (size_t)a->hdim * 4, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(f->norm_ptr(li, 3), L.k_norm, (size_t)a->hdim * 4, hipMemcpyHostToDevice));
+        put(f->norm_ptr(li, 0), L.attn_norm, H);
+        put(f->norm_ptr(li, 1), L.ffn_norm, H);
+        put(f->norm_ptr(li, 2), L.q_norm, D);
+        put(f->norm_ptr(li, 3), L.k_norm, D);
+    }
+    put(f->out_norm, a->out_norm, H);
+    put(f->rope_c, a->rope_cos, rb);
+    put(f->rope_s, a->rope_sin, rb);
+    if (changed || !ok) f->par_sent = false;
+    if (!ok) {
+        set_err(c, "fused_prepare: a norm or RoPE table is missing");
+        c->broken = true;
+        return false;
+    }
+    if (changed) {
+        HIPCHK(c, hipStreamSynchronize(c->s));  // steps in flight read the old ones
+        HIPCHK(c, hipMemcpy(f->par, f->par_host.data(), f->par_host.size(), hipMemcpyHostToDevice));
+        f->par_sent = true;
     }
     if (f->eps != a->eps) free_graphs(f);  // captured kernels hold eps by value
     f->eps = a->eps;
@@ -739,14 +770,15 @@ static bool hip_fused_prepare(void* impl, const hymt2_fused_args* a) {
     f->eps = a->eps;
     const size_t B = HY_MAX_CHUNK, H = a->hidden, F = a->ffn, Q = a->qdim, KV = a->kvdim;
     f->in_bytes = kInH + B * H * 4;
+    auto padded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t norm_b = padded((size_t)a->n_layer * (2 * H + 2 * a->hdim) * 4), out_b = padded(H * 4),
+                 rope_b = padded((size_t)a->ctx * a->rope_half * 4 + 4), par_bytes = norm_b + out_b + 2 * rope_b;
     bool ok = dalloc(c, &f->in_dev, f->in_bytes) && hipHostMalloc(&f->in_host, f->in_bytes, 0) == hipSuccess;
     ok = ok && dalloc(c, &f->q, B * Q * 4) && dalloc(c, &f->k, B * KV * 4) && dalloc(c, &f->v, B * KV * 4) &&
          dalloc(c, &f->ao, B * Q * 4) && dalloc(c, &f->g, B * F * 4) && dalloc(c, &f->u, B * F * 4) &&
          dalloc(c, &f->act_h, B * (H / 256) * sizeof(HyQ8K)) && dalloc(c, &f->act_q, B * (Q / 256) * sizeof(HyQ8K)) &&
          dalloc(c, &f->act_f, B * (F / 256) * sizeof(HyQ8K)) &&
-         dalloc(c, &f->rope_c, (size_t)a->ctx * a->rope_half * 4 + 4) &&
-         dalloc(c, &f->rope_s, (size_t)a->ctx * a->rope_half * 4 + 4) && dalloc(c, &f->out_norm, H * 4) &&
-         dalloc(c, &f->norms, (size_t)a->n_layer * (2 * H + 2 * a->hdim) * 4) &&
+         dalloc(c, &f->par, par_bytes) &&
          dalloc(c, &f->kc, (size_t)a->n_layer * a->ctx * KV * 2) &&
          dalloc(c, &f->vc, (size_t)a->n_layer * a->ctx * KV * 2) && dalloc(c, &f->slots, (size_t)kArgSlots * 8) &&
          dalloc(c, &f->sc, (size_t)a->heads * split_sc_stride(a->ctx) * 4) &&
@@ -758,6 +790,11 @@ static bool hip_fused_prepare(void* impl, const hymt2_fused_args* a) {
         free_fused(f);
         return false;
     }
+    f->norms = reinterpret_cast<float*>(f->par);
+    f->out_norm = reinterpret_cast<float*>(f->par + norm_b);
+    f->rope_c = reinterpret_cast<float*>(f->par + norm_b + out_b);
+    f->rope_s = reinterpret_cast<float*>(f->par + norm_b + out_b + rope_b);
+    f->par_host.assign(par_bytes, 0);
     f->d_pos = reinterpret_cast<int*>(f->in_dev);
     f->d_rope = reinterpret_cast<float*>(f->in_dev + 64);
     f->d_h = reinterpret_cast<float*>(f->in_dev + kInH);
@@ -1217,11 +1254,11 @@ int hymt2_hip_attn_split_from(void* impl, int from) {
 // Begins a device loop over positions 0 .. n_total - 1 whose first keep positions (keep <
 // n_prompt) already hold the prompt's K/V; stop ids (at most kStopIds) are recorded by k_finish.
 static int gen_begin_at(Ctx* c, const hymt2_fused_args* shape, hy_dweight* embd, int vocab_out, const int* prompt,
-                        int n_prompt, int n_total, int keep, const int* stop_ids, int n_stop) {
+                        int n_prompt, int n_total, int keep, const int* stop_ids, int n_stop, bool prepared = false) {
     if (!c || c->broken || !shape || !prompt || n_prompt < 1 || n_total <= n_prompt || keep < 0 || keep >= n_prompt ||
         n_stop < 0 || n_stop > kStopIds || (n_stop && !stop_ids))
         return -1;
-    if (!hip_fused_prepare(c, shape)) return -2;
+    if (!prepared && !hip_fused_prepare(c, shape)) return -2;
     Fused* f = c->f;
     f->gen_total = 0;
     const DW* e = dw(embd);
@@ -1289,7 +1326,7 @@ static int gen_begin_at(Ctx* c, const hymt2_fused_args* shape, hy_dweight* embd,
     for (int j = 0; j < kStopIds; j++) stv[j] = j < n_stop ? stop_ids[j] : -1;
     stv[kStopIds] = INT_MAX;
     *f->stop_host = INT_MAX;
-    memset(f->in_host, 0, f->in_bytes);
+    memset(f->in_host, 0, kInH);
     stage_pos(f, shape, keep);
     if (hipMemcpyAsync(f->ids, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice, c->s) != hipSuccess ||
         hipMemcpyAsync(f->stop, stv, sizeof stv, hipMemcpyHostToDevice, c->s) != hipSuccess ||
@@ -1631,7 +1668,7 @@ int hymt2_hip_generate_ids(void* impl, const hymt2_fused_args* shape, hy_dweight
         while (keep < f->cache_n && keep < n_prompt - 1 && f->cache_tok[keep] == prompt[keep]) keep++;
     f->cache_n = 0;  // until this loop has finished
     int rc = gen_begin_at(c, shape, embd, vocab_out, prompt, n_prompt, n_prompt + max_tokens, keep,
-                          n_stop ? opts->stop_ids : nullptr, n_stop);
+                          n_stop ? opts->stop_ids : nullptr, n_stop, true);
     if (rc) return rc;
     (void)hipEventRecord(c->ev[0], c->s);
     if ((rc = chunk > 1 ? hymt2_hip_gen_prefill(impl, shape, chunk) : hymt2_hip_gen_steps(impl, n_prompt - keep)))
