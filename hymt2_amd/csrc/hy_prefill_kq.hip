@@ -489,7 +489,9 @@ hipError_t kq_split(GemmLaunchT<NJ>& L, hipStream_t s) {
 //   48 tokens: gate/up 19.0 split, 21.0 whole; down 15.7 split in 2 token tiles, 18.8 in 1
 //   72 tokens: gate/up 21.6 in 1 token tile, 23.3 in 4; down 18.7 in 2 rows' tiles, 20.5 in 1
 //   128 tokens: gate/up 23.3 in 4 token tiles, 25.5 in 2, 32 in 1 or split (304); qkv 12.1 in 2,
-//   13.3 split, 15.8 in 1 (108); down 20.9 in 2 x 2 tiles split, 24.2 in 1 x 2, 30 whole (189)
+//   13.3 split, 15.8 in 1 (108); down 20.9 in 2 x 2 tiles split, 24.2 in 1 x 2, 30 whole (189);
+//   alone: 512 rows of Q4_K 5.1 split, 7.4 whole, of Q6_K 5.9 and 9.8 (2048 rows of Q4_K 10.0 and 7.7);
+//   6144 rows of Q4_K 12.7 in 4 token tiles and K halves, 13.7 with K whole
 template <int Q, int NJ, bool PAIR>
 hipError_t kq_shape(GemmLaunchT<NJ>& L, hipStream_t s) {
     int rows = 0;
@@ -504,9 +506,13 @@ hipError_t kq_shape(GemmLaunchT<NJ>& L, hipStream_t s) {
         if (tt >= 3 && wgs >= (PAIR ? 512 : 256)) return kq_go<Q, NJ, 4, 4, 1, 1, PAIR>(L, s);
         return tt > 1 ? kq_go<Q, NJ, 2, 4, 1, 1, PAIR>(L, s) : kq_go<Q, NJ, 1, 4, 1, 1, PAIR>(L, s);
     }
-    if (L.nb <= 32 && (tt == 1 || (PAIR && tt <= 3 && L.nb <= 8))) return kq_split<Q, NJ, 1, 1, PAIR>(L, s);
+    const int tiles = (rows + 15) / 16 * tt;
+    if (L.nb <= 32 && (tt == 1 || (PAIR && tt <= 3 && L.nb <= 8) || (!PAIR && tiles <= 384)))
+        return kq_split<Q, NJ, 1, 1, PAIR>(L, s);
     if constexpr (!PAIR)
         if (L.nb <= 32 && L.nb >= 12) return tt <= 3 ? kq_split<Q, NJ, 2, 1, false>(L, s) : kq_split<Q, NJ, 2, 2, false>(L, s);
+    if constexpr (!PAIR)
+        if (tt >= 6 && rows >= 4096 && L.nb <= 8) return kq_go<Q, NJ, 4, 4, 2, 4, false>(L, s);
     if (tt >= 6 && rows >= 4096) return kq_go<Q, NJ, 4, 4, 1, 1, PAIR>(L, s);
     if (tt >= 6 && rows > 2048) return kq_go<Q, NJ, 2, 4, 1, 1, PAIR>(L, s);
     return kq_go<Q, NJ, 1, 4, 1, 1, PAIR>(L, s);
