@@ -267,7 +267,7 @@ hipError_t launch_attention(const PipeAttn& J, int rows, hipStream_t s);
 hipError_t launch_rmsnorm_q8k(const PipeNorm& J, int rows, hipStream_t s);  // hidden 2048 only
 hipError_t launch_quantize_q8k(const PipeQuant& J, int rows, hipStream_t s);
 
-// Single-token attention, one workgroup per query head (k_attn1, hy_attn_decode.hip): RoPE
+// Single-token attention, one or two workgroups per query head (k_attn1, hy_attn_decode.hip): RoPE
 // and RMSNorm of q and k, the bf16 KV store at the position, softmax attention over positions
 // 0..pos, fp32 output row per head into ao (quantized by the o-projection).
 constexpr int kA1MaxCtx = 4096;

@@ -126,8 +126,8 @@ HYMT2_HIP_API void *hymt2_hip_stream(void *impl);
  * 0 on success, negative on error):
  *   quantize_q8k: x[nt][k] fp32 -> act[nt][k/256] q8k_block (quantize_q8k, src/kernels.c:128)
  *   matvec:       out[t*n + r] = row r of an uploaded weight . act[t] (matmul_rows,
- *                 src/kernels.c:1241), panel / Q4_K / Q6_K weights, 1 <= nt <= 128; above 16
- *                 tokens panel weights run on the int8-MFMA GEMM */
+ *                 src/kernels.c:1241), panel / Q4_K / Q6_K weights, 1 <= nt <= 128; from
+ *                 5 tokens (Q4_K / Q6_K: 4) on the int8-MFMA GEMM */
 HYMT2_HIP_API int hymt2_hip_quantize_q8k(void *impl, const float *x_dev, void *act_dev, int k, int nt);
 HYMT2_HIP_API int hymt2_hip_matvec(void *impl, hy_dweight *w, const void *act_dev, float *out_dev, int nt);
 
@@ -230,7 +230,7 @@ HYMT2_HIP_API int hymt2_hip_generate_ids(void *impl, const hymt2_fused_args *sha
 /* Single-token attention form by position (no counterpart in the reference interface): a forward
  * at position >= from (fused_forward with nt == 1, and the device loop's steps) runs the split
  * attention, whose scores use many CUs (k_attn_scores, then k_attn_out); positions below run
- * the one-workgroup-per-head kernel (k_attn1). Both give the same bits. from < 0 restores the
+ * the whole-row kernel (k_attn1, one or two workgroups a head). Both give the same bits. from < 0 restores the
  * default. Shapes k_attn1 does not take (head dim other than 64/128, ctx > 4096) always split.
  * Drops the captured graphs (and ends a device loop in progress). 0 on success. */
 HYMT2_HIP_API int hymt2_hip_attn_split_from(void *impl, int from);
@@ -240,7 +240,8 @@ HYMT2_HIP_API int hymt2_hip_attn_split_from(void *impl, int from);
  * several chunks runs pipelined over the layers: chunk i's layer l in the same launches as
  * chunk i + 1's layer l - 1, up to depth chunks at a time. Every chunk is the same forward over
  * the same KV cache as in the one-after-another order, so the results are the same bits.
- * Applies to panel-weight models with hidden 2048 and the chunk attention kernel's shapes;
+ * Applies to models with hidden 2048 and the chunk attention kernel's shapes whose quantized weights
+ * are of one GEMM (panels, or Q4_K / Q6_K) in each place and whose gates and ups are of one kind;
  * others run one chunk after another. depth 1 turns it off; depth < 1 only queries. Default
  * and maximum 8. Returns the previous depth, or -1 without a context. */
 HYMT2_HIP_API int hymt2_hip_prefill_pipeline(void *impl, int depth);
