@@ -403,7 +403,10 @@ static bool build_launch(const JobSpec* js, int njobs, bool pair, int nt, int th
             const MvWeight& m = js[j].w->mw;
             const int spr = m.nb * mv_segments_per_block(m.kind) * (pair ? 2 : 1);
             const int rpw = (threads * segs) / spr;
-            if (rpw < 1) ok = false;
+            if (rpw < 1) {  // a row of more segments than the workgroup takes (K above 8192 at 256 Q4_K segments)
+                ok = false;
+                break;
+            }
             L.job[j].rows_per_wg = rpw;
             L.job[j].wg_begin = wgs;
             if (!pair || j == 0) wgs += (m.n + rpw - 1) / rpw;

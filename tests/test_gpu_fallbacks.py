@@ -10,15 +10,17 @@ against the oracle, bit for bit (src/model.c:767-795, :857-876, :887-900):
   chunks;
 * a quantized (Q6_K / Q4_K) LM head at hidden 1024: the decode matvec with the argmax epilogue
   takes K = 2048 and 6144 only, so the head runs on the general matvec with the RMSNorm + Q8_K
-  prologue and a separate argmax kernel (k_argmax over the logits).
+  prologue and a separate argmax kernel (k_argmax over the logits);
+* contractions of rows longer than 8192 (Q4_K, Q6_K) or 16384 (panels) weights.
 
-Each test compares the logits of the reference host's boundary (fused_forward per chunk) and the
+Each model test compares the logits of the reference host's boundary (fused_forward per chunk) and the
 device loop's greedy ids with the oracle's."""
 import numpy as np
 import pytest
 
 from hymt2_amd import abi, lib, synth
 from oracle import oracle as O
+from test_gpu_kernels import run_matvec
 
 pytestmark = pytest.mark.gpu
 
@@ -99,3 +101,27 @@ def test_quantized_head_hidden_1024(backend, head):
     model = synth.make_model(shape, mode="stq", seed=98 + head, head_type=head)
     prompt = synth.rand_prompt(synth.rng(99), 21, shape.vocab)
     check_model(backend, model, prompt, 12, batches=(16, 1), chunks=(1, 8))
+
+
+@pytest.mark.parametrize("gt,k", [(abi.GT_Q4_K, 8192), (abi.GT_Q4_K, 8448), (abi.GT_Q6_K, 16640), (abi.GT_Q4_K, 32768),
+                                  (abi.GT_STQ1_0, 16384), (abi.GT_STQ1_0, 16640), (abi.GT_Q2_0C, 33280)])
+def test_long_rows(backend, gt, k):
+    """Rows around and past the segments a 256-thread workgroup of the general matvec takes at one a
+    thread (32 blocks of Q4_K and Q6_K, 64 of a panel), up to four a thread (128 blocks of Q4_K), at
+    the token counts it serves."""
+    g = synth.rng(gt + k)
+    w = synth.make_weight(g, gt, 19, k)
+    for nt in (1, 2, 3):
+        x = synth.activations(g, nt, k)
+        out, xq = run_matvec(backend, w, x)
+        assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, nt))), f"nt={nt}"
+
+
+def test_rows_past_the_general_matvec(backend):
+    """One block past its longest row: refused, and the context goes on."""
+    g = synth.rng(33024)
+    with pytest.raises(RuntimeError):
+        run_matvec(backend, synth.make_weight(g, abi.GT_Q4_K, 3, 33024), synth.activations(g, 1, 33024))
+    w, x = synth.make_weight(g, abi.GT_Q4_K, 3, 32768), synth.activations(g, 1, 32768)
+    out, xq = run_matvec(backend, w, x)
+    assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, 1)))
