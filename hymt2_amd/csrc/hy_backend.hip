@@ -104,7 +104,8 @@ struct Fused {
     int* stop_host_dev = nullptr;
     // the ids whose K/V the cache holds after the last hymt2_hip_generate_ids call (positions
     // 0 .. cache_n - 1), and what they were computed with; any other writer of the cache
-    // (fused_forward, the other device-loop entry points) sets cache_n to 0
+    // (fused_forward, the other device-loop entry points) sets cache_n to 0, as do a changed
+    // parameter (copy_params) and the release of one of the weights
     std::vector<int> cache_tok;
     int cache_n = 0;
     std::vector<const void*> cache_sig;
@@ -339,13 +340,16 @@ static hy_dweight* hip_upload(void* impl, const hymt2_weight* w) {
 static void free_graphs(Fused* f);
 
 // Frees a device weight. The context's captured graphs may name it (their signatures hold
-// weight handles, and a later upload can reuse the address), so they are dropped too.
+// weight handles, and a later upload can reuse the address), so they are dropped too, as is the
+// prefix record of K/V formed with it.
 static void hip_release(hy_dweight* w) {
     DW* d = reinterpret_cast<DW*>(w);
     if (!d) return;
     if (d->c && d->c->f) {
         if (d->c->s) (void)hipStreamSynchronize(d->c->s);
-        free_graphs(d->c->f);
+        Fused* f = d->c->f;
+        free_graphs(f);
+        if (std::find(f->cache_sig.begin(), f->cache_sig.end(), w) != f->cache_sig.end()) f->cache_n = 0;
     }
     if (d->mem) (void)hipFree(d->mem);
     if (d->op_host) (void)hipHostFree(d->op_host);
@@ -736,6 +740,7 @@ static bool copy_params(Ctx* c, const hymt2_fused_args* a) {
         return false;
     }
     if (changed) {
+        f->cache_n = 0;  // K/V formed with the old values (the record's key holds the arrays' addresses)
         HIPCHK(c, hipStreamSynchronize(c->s));  // steps in flight read the old ones
         HIPCHK(c, hipMemcpy(f->par, f->par_host.data(), f->par_host.size(), hipMemcpyHostToDevice));
         f->par_sent = true;
