@@ -492,6 +492,15 @@ hipError_t kq_split(GemmLaunchT<NJ>& L, hipStream_t s) {
 //   13.3 split, 15.8 in 1 (108); down 20.9 in 2 x 2 tiles split, 24.2 in 1 x 2, 30 whole (189);
 //   alone: 512 rows of Q4_K 5.1 split, 7.4 whole, of Q6_K 5.9 and 9.8 (2048 rows of Q4_K 10.0 and 7.7);
 //   6144 rows of Q4_K 12.7 in 4 token tiles and K halves, 13.7 with K whole
+// Single contractions of 12-32 blocks are split, in the form with the fewest tokens and rows a
+// workgroup whose workgroups the CUs take at once (256 of the 256- and 512-thread ones run side by
+// side; more take turns). 2048 x 6144 alone, Q4_K / Q6_K: 32 tokens 8.1 / 10.3 in 1 token tile (256
+// workgroups), 10.8 / 12.6 in 2 (128); 48 tokens 12.2 / 16.0 in 1 (384), 11.3 / 12.7 in 2 (256); 64
+// tokens 12.2 / 16.3 in 1 (512), 11.3 / 12.9 in 2 (256), 13.1 / 16.8 in 2 x 2 (128); 80 tokens 16.2 /
+// 18.8 in 2 (384), 13.3 / 16.6 in 2 x 2 (192). 2560 x 6912 at 48 tokens: 18.2 / 21.3 in 2 (320), 14.2 /
+// 18.1 in 2 x 2 (160); 4112 x 3840, where no form fits at once, 16.1 / 18.2 in 2 (514), 16.4 / 20.0 in
+// 2 x 2 (258). With fewer blocks the steps are few and 384 workgroups of 1 token tile are as
+// fast: 2048 x 2048 at 48 tokens 6.8 / 8.1 in 1, 7.0 / 7.5 in 2, 7.9 / 11.0 with K whole.
 template <int Q, int NJ, bool PAIR>
 hipError_t kq_shape(GemmLaunchT<NJ>& L, hipStream_t s) {
     int rows = 0;
@@ -506,11 +515,15 @@ hipError_t kq_shape(GemmLaunchT<NJ>& L, hipStream_t s) {
         if (tt >= 3 && wgs >= (PAIR ? 512 : 256)) return kq_go<Q, NJ, 4, 4, 1, 1, PAIR>(L, s);
         return tt > 1 ? kq_go<Q, NJ, 2, 4, 1, 1, PAIR>(L, s) : kq_go<Q, NJ, 1, 4, 1, 1, PAIR>(L, s);
     }
-    const int tiles = (rows + 15) / 16 * tt;
-    if (L.nb <= 32 && (tt == 1 || (PAIR && tt <= 3 && L.nb <= 8) || (!PAIR && tiles <= 384)))
+    const int rt = (rows + 15) / 16, tiles = rt * tt;
+    if (L.nb <= 32 && (tt == 1 || (PAIR && tt <= 3 && L.nb <= 8) || (!PAIR && tiles <= (L.nb < 12 ? 384 : 256))))
         return kq_split<Q, NJ, 1, 1, PAIR>(L, s);
     if constexpr (!PAIR)
-        if (L.nb <= 32 && L.nb >= 12) return tt <= 3 ? kq_split<Q, NJ, 2, 1, false>(L, s) : kq_split<Q, NJ, 2, 2, false>(L, s);
+        if (L.nb <= 32 && L.nb >= 12) {
+            const int t2 = (tt + 1) / 2;
+            const bool one_row = rt * t2 <= 256 || (tt <= 3 && (rt + 1) / 2 * t2 > 256);
+            return one_row ? kq_split<Q, NJ, 2, 1, false>(L, s) : kq_split<Q, NJ, 2, 2, false>(L, s);
+        }
     if constexpr (!PAIR)
         if (tt >= 6 && rows >= 4096 && L.nb <= 8) return kq_go<Q, NJ, 4, 4, 2, 4, false>(L, s);
     if (tt >= 6 && rows >= 4096) return kq_go<Q, NJ, 4, 4, 1, 1, PAIR>(L, s);

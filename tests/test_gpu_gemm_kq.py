@@ -4,7 +4,8 @@ Cases sit at the edges of its tiles and splits: token counts around 16-token til
 where the split changes, row counts that end inside a 16-row tile, K from one block to past the
 largest that is split over wavefronts (33 blocks), and extreme block contents (every scale, min,
 code and activation at its largest magnitude, of either sign, where the int8 digits of the scaled
-weights and the f16 products of mins and bsums reach their bounds)."""
+weights and the f16 products of mins and bsums reach their bounds). The sizes at which each form of
+the launch is chosen follow kq_shape's rules; SPLITS names the form each of its cases takes."""
 import numpy as np
 import pytest
 
@@ -51,6 +52,31 @@ def test_gemm_kq_vs_oracle(backend, gt, n, k):
             x[1::4] = 1.0               # and bsums at their largest
         out, xq = run_matvec(backend, w, x)
         assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, nt))), f"nt={nt}"
+
+
+# 12 to 32 blocks alone: (rows, K, tokens) and the form: token tiles x row tiles a workgroup of each K set
+SPLITS = [
+    (2048, 3328, 33),   # 2 x 1, four blocks a set, the last set's short (13 of 16); 128 row tiles
+    (2000, 5120, 47),   # 2 x 1, six blocks a set (20 of 24), ragged rows
+    (2048, 6144, 48),   # 2 x 1, full sets (24 blocks)
+    (2041, 6144, 64),   # 2 x 1, four token tiles
+    (800, 7168, 81),    # 2 x 1, eight blocks a set (28 of 32), six token tiles
+    (2560, 3072, 48),   # 2 x 2, three token tiles
+    (2048, 3328, 65),   # 2 x 2, five token tiles
+    (2017, 6144, 128),  # 2 x 2, an odd number of row tiles
+    (4112, 3840, 17),   # 2 x 2, more row tiles than 256
+    (4112, 3072, 33),   # 2 x 1, more workgroups of either form than 256
+]
+
+
+@pytest.mark.parametrize("gt", [abi.GT_Q4_K, abi.GT_Q6_K])
+@pytest.mark.parametrize("n,k,nt", SPLITS)
+def test_split_contractions(backend, gt, n, k, nt):
+    g = synth.rng(gt * 17 + n + k + nt)
+    w = raw_weight(g, gt, n, k, False)
+    x = synth.activations(g, nt, k)
+    out, xq = run_matvec(backend, w, x)
+    assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, nt)))
 
 
 def test_gemm_kq_in_a_model(backend):
