@@ -484,9 +484,10 @@ static bool run_mv1(Ctx* c, const JobSpec* js, int njobs, bool pair, const MvOpt
 }
 
 // Several tokens: the int8-MFMA GEMM of the panel formats or of Q4_K / Q6_K from kGemmMinTokens + 1
-// tokens (the reference host's 16-token batches among them); below that, and for groups that mix
-// panels with the others, the general matvec kernel runs over groups of at most HY_MAX_BATCH
-// tokens. All give every token the single-token result. The threshold as measured on panels (a fused_forward of the config-3 model, matvec
+// tokens (the reference host's 16-token batches among them); below that, for few or long rows of
+// Q4_K / Q6_K (kq_matvec), and for groups that mix panels with the others, the general matvec kernel
+// runs over groups of at most HY_MAX_BATCH tokens. All give every token the single-token result. The
+// threshold as measured on panels (a fused_forward of the config-3 model, matvec
 // against GEMM: 16 tokens 3.27 -> 1.95-2.01 ms, 8 tokens 2.34 -> 1.91-1.97, 4 tokens equal,
 // 2 tokens 1.71-1.78 against 1.87-1.92 ms). Q4_K / Q6_K one token earlier (16 layers of a Q4_K_M
 // model: 2 tokens 965 against 1010 us, 3 tokens 1037 against 1019, 4 tokens 1110 against 1031; one
@@ -494,8 +495,31 @@ static bool run_mv1(Ctx* c, const JobSpec* js, int njobs, bool pair, const MvOpt
 constexpr int kGemmMinTokens = 4;
 constexpr int kGemmKqMinTokens = 3;
 
+// Whether the general matvec is the faster one for a contraction of one of Q4_K and Q6_K at up to
+// HY_MAX_BATCH tokens. The GEMM's time is its block steps (K over four sets of wavefronts up to 32
+// blocks, whole beyond), whatever the rows; the matvec's grows with the tokens, and past a few hundred
+// workgroups with the rows. The two sides below are both kernels' us, fitted to 90 sizes of 16-3072 rows
+// by 256-14336 weights at 4-16 tokens; of the 1620 pairs of times the slower kernel is picked, by more
+// than 3 %, at 20. Matvec and GEMM at 4, 8 and 16 tokens: 512 x 2048 of Q6_K 4.2, 5.6, 8.3 and 5.3-5.4;
+// 512 x 6144 of Q6_K 5.5, 7.2, 10.5 and 9.5-9.9; 2048 x 2048 of Q4_K 5.3, 7.1, 10.1 and 5.2-5.3;
+// 1024 x 14336 of Q4_K 10.5, 15.5, 25.0 and 31.7-32.1.
+static bool kq_matvec(const JobSpec* js, int njobs, int nt) {
+    if (nt > HY_MAX_BATCH) return false;
+    float blocks = 0.f;
+    for (int j = 0; j < njobs; j++) {
+        const MvWeight& W = js[j].w->mw;
+        if (W.kind != js[0].w->mw.kind) return false;  // mixed: q, k, v of 1536-3072 rows 1-13 % faster by GEMM from 4 tokens
+        blocks += (float)W.n * (float)W.nb;
+    }
+    const int nb = js[0].w->mw.nb, steps = nb > 32 ? nb : std::max(2, (nb + 7) / 8 * 2);
+    const float step = js[0].w->mw.kind == KIND_Q6K ? 0.9f : nb > 32 ? 0.5f : 0.6f;
+    const float token = std::max(nb > 32 ? 0.7f : 0.35f, blocks / 40000.f);
+    return 2.7f + blocks / 18000.f + (float)nt * token < 3.3f + (float)steps * step + blocks / 60000.f;
+}
+
 static bool run_multi(Ctx* c, const JobSpec* js, int njobs, bool pair, int nt, const MvOpts& o) {
-    if (nt > (js[0].w->mw.kind == KIND_PANEL ? kGemmMinTokens : kGemmKqMinTokens) && o.pro == PRO_NONE) {
+    const bool panel = js[0].w->mw.kind == KIND_PANEL;
+    if (nt > (panel ? kGemmMinTokens : kGemmKqMinTokens) && o.pro == PRO_NONE && (panel || !kq_matvec(js, njobs, nt))) {
         GemmLaunch G;
         memset(&G, 0, sizeof G);
         G.njobs = njobs;

@@ -127,7 +127,7 @@ HYMT2_HIP_API void *hymt2_hip_stream(void *impl);
  *   quantize_q8k: x[nt][k] fp32 -> act[nt][k/256] q8k_block (quantize_q8k, src/kernels.c:128)
  *   matvec:       out[t*n + r] = row r of an uploaded weight . act[t] (matmul_rows,
  *                 src/kernels.c:1241), panel / Q4_K / Q6_K weights, 1 <= nt <= 128; from
- *                 5 tokens (Q4_K / Q6_K: 4) on the int8-MFMA GEMM */
+ *                 5 tokens (Q4_K / Q6_K: 4, few or long rows 5 to 17) on the int8-MFMA GEMM */
 HYMT2_HIP_API int hymt2_hip_quantize_q8k(void *impl, const float *x_dev, void *act_dev, int k, int nt);
 HYMT2_HIP_API int hymt2_hip_matvec(void *impl, hy_dweight *w, const void *act_dev, float *out_dev, int nt);
 

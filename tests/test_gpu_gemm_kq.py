@@ -1,7 +1,7 @@
 """The Q4_K / Q6_K GEMM (k_gemm_kq) against the oracle, bit for bit.
 
-Cases sit at the edges of its tiles and splits: token counts around 16-token tiles and the counts
-where the split changes, row counts that end inside a 16-row tile, K from one block to past the
+Cases sit at the edges of its tiles and splits: token counts around 16-token tiles, the counts
+where the split changes and those up to 16 where few or long rows stay on the general matvec, row counts that end inside a 16-row tile, K from one block to past the
 largest that is split over wavefronts (33 blocks), and extreme block contents (every scale, min,
 code and activation at its largest magnitude, of either sign, where the int8 digits of the scaled
 weights and the f16 products of mins and bsums reach their bounds). The sizes at which each form of
@@ -43,7 +43,7 @@ def raw_weight(g, gt, n, k, extreme):
                                  (48, 6144), (31, 8192), (40, 8448), (4100, 512), (2200, 256)])
 def test_gemm_kq_vs_oracle(backend, gt, n, k):
     g = synth.rng(gt * 13 + n + k)
-    for nt in (5, 16, 17, 48, 49, 80, 81, 128):
+    for nt in (4, 5, 8, 16, 17, 48, 49, 80, 81, 128):
         extreme = nt in (16, 49, 128)
         w = raw_weight(g, gt, n, k, extreme)
         x = synth.activations(g, nt, k)
