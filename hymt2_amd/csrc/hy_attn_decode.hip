@@ -32,10 +32,10 @@ constexpr int kA1Waves = kA1Threads / 64;
 constexpr int kA1Tile = 96;            // positions per product tile
 constexpr int kA1Prod = kA1Threads - 128;  // producer threads (wavefronts 2-7)
 constexpr int kA1Chunk = 32;           // positions per chain step (16 LDS reads of 2 products)
-constexpr int kA1SerialSum = 256;      // softmax rows up to this length: the lane-serial sum
 constexpr int kA1PairRow = kA1Threads / 2;  // rows up to this length: two lanes per key
-static_assert(kA1SerialSum <= kA1PairRow, "the serial sum reads the pair form's padded exponentials");
-constexpr int kA1ShortRow = kA1PairRow;     // rows up to this length: V staged whole, direct chains
+// rows up to this length: the lane-serial sum (of the pair form's padded exponentials), V staged whole
+// meanwhile, direct chains
+constexpr int kA1ShortRow = kA1PairRow;
 
 __device__ __forceinline__ void bf16x8f(const uint4& v, float* f) {
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -364,7 +364,6 @@ struct A1Smem {
     alignas(16) uint16_t kb[HD];
     alignas(16) uint16_t vb[HD];
     float red[kA1Waves];
-    float stat;
     uint64_t etab[32];  // expf table
 };
 
@@ -475,7 +474,6 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
     // 3. softmax (src/model.c:781-789): max (order-free), e_j = expf(s_j - max), their sum in
     //    position order, inv = 1 / sum. Short rows: the lane-serial chain of wavefront 0; long
     //    ones: the exact segmented form over 8 consecutive positions per thread.
-    float inv;
     {
         float mx = red[0];
 #pragma unroll
@@ -494,21 +492,16 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
             if (j < n) ex[j] = hy_expf_tab(sv[p] - mx, S.etab);
         }
         hy_lds_barrier();
-        if (n <= kA1SerialSum) {
-            if (wave == 0) {
-                const float sum = hy_wave_seq_sum(ex, (n + 31) / 32 * 32, lane);  // the same value in every lane
-                if (lane == 0) S.stat = 1.0f / sum;
-                if (n <= kA1ShortRow) {  // short rows: p_j = e_j * (1 / sum) in place, once per position
-                    const float iv = 1.0f / sum;
-                    for (int j = lane; j < n; j += 64) ex[j] = ex[j] * iv;
-                }
-            } else if (n <= kA1ShortRow && prd) {  // meanwhile the producers stage V whole
+        if (n <= kA1ShortRow) {
+            if (wave == 0) {  // p_j = e_j * (1 / sum) in place, once per position
+                const float iv = 1.0f / hy_wave_seq_sum(ex, (n + 31) / 32 * 32, lane);  // the same value in every lane
+                for (int j = lane; j < n; j += 64) ex[j] = ex[j] * iv;
+            } else if (prd) {  // meanwhile the producers stage V whole
                 a1_stage_v<VD>(v0, S.stage, vb, 0, pp, pos, n);
                 if (n > kA1Tile) a1_stage_v<VD>(v1, S.stage, vb, kA1Tile, pp, pos, n);
                 if (n > 2 * kA1Tile) a1_stage_v<VD>(v2, S.stage, vb, 2 * kA1Tile, pp, pos, n);
             }
             hy_lds_barrier();
-            inv = S.stat;
         } else {
             const int e0 = 8 * tid;
             float e[8];
@@ -521,9 +514,7 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
 #pragma unroll
                 for (int i = 0; i < 8; i++) e[i] = e0 + i < n ? ev[i] : 0.f;
             }
-            inv = 1.0f / hy_block_exact_sum8<kA1Waves, false>(e, S.exs, wave, lane);
-        }
-        if (n > kA1ShortRow) {
+            const float inv = 1.0f / hy_block_exact_sum8<kA1Waves, false>(e, S.exs, wave, lane);
             // p_j = e_j * (1 / sum), once per position; +0 past the row to the end of its last tile
             const int end = (n + kA1Tile - 1) / kA1Tile * kA1Tile;
             for (int j = tid; j < end; j += kA1Threads) ex[j] = j < n ? ex[j] * inv : 0.f;
@@ -532,12 +523,12 @@ __device__ __forceinline__ void a1_core(const Attn1Args& a, A1Smem<HD>& S, const
     }
 
     // 4. o[d] = sum_j p_j * V_j[d] in position order (axpy_bf16). Barrier t: tile t is in
-    //    buffer t % 2, and tile t - 1's buffer has been read. Wavefronts 0 .. HD/64 - 1 walk tile
-    //    t after barrier t; the producers convert tile t's V rows before it, with V three tiles
-    //    ahead, in groups of three steps (one loop exit; steps past the row only load).
-    // Short rows: every lane of wavefronts 0 .. HD/64 - 1 walks its dimension over the staged V.
+    //    buffer t % 2, and tile t - 1's buffer has been read. Wavefront 0, one dimension a lane,
+    //    walks tile t after barrier t; the producers convert tile t's V rows before it, with V three
+    //    tiles ahead, in groups of three steps (one loop exit; steps past the row only load).
+    // Short rows: every lane of wavefront 0 walks its dimension over the staged V.
     if (n <= kA1ShortRow) {
-        static_assert(kA1ShortRow <= kA1SerialSum && kA1ShortRow <= 3 * kA1Tile, "three tiles of V, one sum");
+        static_assert(kA1ShortRow <= 3 * kA1Tile && VD == 64, "three tiles of V, one wavefront of dimensions");
         if (tid < VD) a.ao[(size_t)h * HD + part * VD + tid] = a1_short_chain<VD>(S.stage + tid, ex, n);
         return;
     }
