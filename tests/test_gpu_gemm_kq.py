@@ -12,7 +12,7 @@ import pytest
 from conftest import ROOT  # noqa: F401  (sys.path)
 from hymt2_amd import abi, lib, synth
 from oracle import oracle as O
-from test_gpu_fallbacks import check_model
+from test_gpu_fallbacks import check_model, oracle_logits
 from test_gpu_kernels import bits, run_matvec
 
 pytestmark = pytest.mark.gpu
@@ -79,9 +79,95 @@ def test_split_contractions(backend, gt, n, k, nt):
     assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, nt)))
 
 
+# up to 11 blocks alone, more than 4096 rows and more than 80 tokens: K halves of four blocks up to
+# eight, whole beyond
+WIDE = [(4100, 2048, 81), (4100, 2048, 128), (4100, 1280, 81), (4096, 1024, 96), (4100, 2560, 81)]
+
+
+@pytest.mark.parametrize("gt", [abi.GT_Q4_K, abi.GT_Q6_K])
+@pytest.mark.parametrize("n,k,nt", WIDE)
+def test_wide_contractions(backend, gt, n, k, nt):
+    """The second K half full (eight blocks), short (five) and empty (four)."""
+    g = synth.rng(gt * 19 + n + k + nt)
+    w = raw_weight(g, gt, n, k, False)
+    x = synth.activations(g, nt, k)
+    out, xq = run_matvec(backend, w, x)
+    assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, nt)))
+
+
+@pytest.mark.parametrize("rows,k,nt", [((512, 128, 128), 2048, 48), ((2048, 1024, 1100), 2048, 81), ((1000, 500, 520), 3328, 40),
+                                       ((1024, 512, 520), 3328, 100), ((2304, 100, 33), 2304, 96), ((1500, 100, 33), 2304, 64)])
+def test_mixed_groups(backend, rows, k, nt):
+    """Q4_K and Q6_K jobs of one launch (a per-op group of two Q4_K weights and a Q6_K one) in each form
+    of the launch: one token tile split, K halves, two token tiles split with one and with two row tiles,
+    two token tiles and one with K whole. Row counts end inside tiles."""
+    g = synth.rng(sum(rows) + k + nt)
+    ws = [raw_weight(g, gt, n, k, False) for n, gt in zip(rows, (abi.GT_Q4_K, abi.GT_Q4_K, abi.GT_Q6_K))]
+    hs = [backend.upload(w) for w in ws]
+    try:
+        x = synth.activations(g, nt, k)
+        xq = O.quantize_q8k(x)
+        for w, out in zip(ws, backend.matmul(hs, [w.n for w in ws], xq, nt)):
+            assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, nt)))
+    finally:
+        for h in hs:
+            backend.release(h)
+
+
+@pytest.mark.parametrize("gt,hidden,ffn", [(abi.GT_Q6_K, 2048, 1024), (abi.GT_Q4_K, 2048, 2304), (abi.GT_Q6_K, 2048, 2304),
+                                           (abi.GT_Q6_K, 2048, 4352), (abi.GT_Q4_K, 2560, 2304), (abi.GT_Q6_K, 2560, 4352)])
+def test_pairs_in_a_model(backend, gt, hidden, ffn):
+    """Gate and up of either kind: split over wavefronts at 16 tokens (eight and ten blocks) and at 48
+    (eight), K whole at 48 (ten) and, in 1, 2 and 4 token tiles by the row count, at 128. Logits after a
+    131-token prompt in batches of each."""
+    shape = synth.ModelShape(n_layer=1, hidden=hidden, ffn=ffn, heads=hidden // 128, kv_heads=4, hdim=128, vocab=300, ctx=140)
+    model = synth.make_model(shape, mode="q4km", seed=191)
+    g = synth.rng(192 + ffn)
+    for nm in ("wg", "wu"):
+        model["layers"][0][nm] = synth.make_weight(g, gt, ffn, hidden)
+    prompt = synth.rand_prompt(synth.rng(193), 131, shape.vocab)
+    ref = oracle_logits(model, prompt)
+    fm = lib.FusedModel(backend, model)
+    try:
+        for batch in (16, 48, 128):
+            assert np.array_equal(bits(fm.prefill(list(prompt), batch=batch)), bits(ref)), f"batch={batch}"
+    finally:
+        fm.close()
+
+
+@pytest.mark.parametrize("gt", [abi.GT_Q4_K, abi.GT_Q6_K])
+def test_pipelined_forms(backend, gt):
+    """Every weight of one kind, four layers and four chunks of a prompt (the last one short): the
+    pipelined launches of one to four chunks in their three forms, pairs and single jobs, against the same
+    chunks one after another, whose launches the tests above compare with the oracle. Ids of the device
+    loop and logits after them."""
+    shape = synth.ModelShape(n_layer=4, hidden=2048, ffn=6144, heads=16, kv_heads=4, hdim=128, vocab=500, ctx=520)
+    model = synth.make_model(synth.ModelShape(**{**shape.__dict__, "ffn": 256}), mode="q4km", seed=201)
+    model["shape"] = shape
+    g = synth.rng(202 + gt)
+    dims = dict(wq=(2048, 2048), wk=(512, 2048), wv=(512, 2048), wo=(2048, 2048), wg=(6144, 2048), wu=(6144, 2048), wd=(2048, 6144))
+    weights = {nm: raw_weight(g, gt, n, k, False) for nm, (n, k) in dims.items()}
+    for L in model["layers"]:
+        L.update(weights)
+    prompt = synth.rand_prompt(synth.rng(203), 500, shape.vocab)
+    fm = lib.FusedModel(backend, model)
+    try:
+        got = []
+        for chunk, depth in ((128, 1), (128, 8), (40, 8), (128, 3)):
+            before = backend.prefill_pipeline(depth)
+            ids, _ = fm.generate_device(prompt, 4, chunk=chunk)
+            got.append((ids, fm.forward([int(ids[-1])], 503, True)))
+            backend.prefill_pipeline(before)
+        assert np.isfinite(got[0][1]).all()
+        for ids, logits in got[1:]:
+            assert np.array_equal(ids, got[0][0]) and np.array_equal(bits(logits), bits(got[0][1]))
+    finally:
+        fm.close()
+
+
 def test_gemm_kq_in_a_model(backend):
-    """Mixed q/k (Q4_K) and v (Q6_K) rows in one launch, gate/up pairs with the SwiGLU epilogue and
-    residual adds, at the 1.8B layer's dimensions and batches that take every split of each."""
+    """Mixed q/k (Q4_K) and v (Q6_K) rows in one launch, Q4_K gate/up pairs with the SwiGLU epilogue and
+    residual adds, at the 1.8B layer's dimensions and at batches of one, three, five and eight token tiles."""
     shape = synth.ModelShape(n_layer=1, hidden=2048, ffn=6144, heads=16, kv_heads=4, hdim=128, vocab=600, ctx=160)
     model = synth.make_model(shape, mode="q4km", seed=171)
     prompt = synth.rand_prompt(synth.rng(172), 150, shape.vocab)
