@@ -149,9 +149,12 @@ struct Ctx {
 
 // Per-op groups whose activations and outputs fit this go through pinned memory of the context: the
 // kernels write the outputs there over PCIe, and a copy kernel brings the activations to the device.
-// Copies to and from the caller's pageable buffers would each wait for the runtime's own staging
-// (a Q4_K gate/up group at one token: 47.5 us with them, 24.1 us without). Larger groups keep the
-// copies: their transfers are worth the DMA engine.
+// Copies to and from the caller's pageable buffers would each wait for the runtime's own staging. The
+// pinned way measured the faster one at every size (us a call of Q4_K_M groups, copies and pinned): q/k/v
+// at 1 token 57.3 and 18.5, at 16 tokens (270 KB) 55.2 and 30.1; gate/up at 1 token 37.7 and 21.0, at 4
+// (215 KB) 48.8 and 30.9, at 8 (430 KB) 57.6 and 40.4, at 16 (860 KB) 77.4 and 59.9, at 32 (1.7 MB) 117
+// and 97, at 128 (6.9 MB) 409 and 365. So the bound is only what a context keeps pinned; it covers the
+// 1.8B model's groups at the host's 16 tokens.
 constexpr size_t kPinBytes = 1u << 20;
 
 // Whether the single-token forward at position pos uses the split attention: long rows, and

@@ -437,7 +437,7 @@ def test_gemm_full_gate_up_vs_single_token(backend):
 
 @pytest.mark.parametrize("gt", [abi.GT_Q4_K, abi.GT_Q6_K])
 def test_multi_token_non_panel_groups(backend, gt):
-    """Q4_K / Q6_K chunks above 16 tokens run the general matvec over groups of 16."""
+    """Q4_K / Q6_K chunks above 16 tokens: three token tiles of their GEMM, the last one ragged."""
     g = synth.rng(gt + 500)
     w = synth.make_weight(g, gt, 300, 2048)
     x = synth.activations(g, 45, 2048)
@@ -446,8 +446,8 @@ def test_multi_token_non_panel_groups(backend, gt):
 
 
 def test_per_op_matmul_128_tokens(backend):
-    """matmul() with a 128-token chunk (a host built with MAX_BATCH = 128): panel weights on the
-    GEMM, a Q6_K weight of the same group on the general kernel."""
+    """matmul() with a 128-token chunk (a host built with MAX_BATCH = 128): panel weights on their
+    GEMM, a Q6_K weight of the same group on its own, a launch each."""
     g = synth.rng(78)
     ws = [synth.make_weight(g, abi.GT_STQ1_0, 512, 1024), synth.make_weight(g, abi.GT_Q2_0C, 256, 1024),
           synth.make_weight(g, abi.GT_Q6_K, 128, 1024)]
@@ -461,6 +461,23 @@ def test_per_op_matmul_128_tokens(backend):
     finally:
         for h in hs:
             backend.release(h)
+
+
+@pytest.mark.parametrize("n", [1904, 1905])
+def test_per_op_matmul_staging_bound(backend, n):
+    """128 tokens of one block and n rows: activations and outputs of 1 MiB, the largest group staged in
+    pinned memory, and one row past it, copied."""
+    g = synth.rng(n)
+    w = synth.make_weight(g, abi.GT_Q4_K, n, 256)
+    x = synth.activations(g, 128, 256)
+    xq = O.quantize_q8k(x)
+    h = backend.upload(w)
+    try:
+        for _ in range(2):
+            out, = backend.matmul([h], [n], xq, 128)
+            assert np.array_equal(bits(out), bits(O.matvec(w, x, xq, 128)))
+    finally:
+        backend.release(h)
 
 
 def test_per_op_weight_out(backend):
