@@ -506,15 +506,16 @@ constexpr int kGemmKqMinTokens = 3;
 // than 3 %, at 20. Matvec and GEMM at 4, 8 and 16 tokens: 512 x 2048 of Q6_K 4.2, 5.6, 8.3 and 5.3-5.4;
 // 512 x 6144 of Q6_K 5.5, 7.2, 10.5 and 9.5-9.9; 2048 x 2048 of Q4_K 5.3, 7.1, 10.1 and 5.2-5.3;
 // 1024 x 14336 of Q4_K 10.5, 15.5, 25.0 and 31.7-32.1.
-static bool kq_matvec(const JobSpec* js, int njobs, int nt) {
-    if (nt > HY_MAX_BATCH) return false;
+static bool kq_matvec(const JobSpec* js, int njobs, bool pair, int nt) {
+    const int nb = js[0].w->mw.nb;
+    if (nt > HY_MAX_BATCH || nb * 8 * (pair ? 2 : 1) > 1024) return false;  // build_launch takes no longer row
     float blocks = 0.f;
     for (int j = 0; j < njobs; j++) {
         const MvWeight& W = js[j].w->mw;
         if (W.kind != js[0].w->mw.kind) return false;  // mixed: q, k, v of 1536-3072 rows 1-13 % faster by GEMM from 4 tokens
         blocks += (float)W.n * (float)W.nb;
     }
-    const int nb = js[0].w->mw.nb, steps = nb > 32 ? nb : std::max(2, (nb + 7) / 8 * 2);
+    const int steps = nb > 32 ? nb : std::max(2, (nb + 7) / 8 * 2);
     const float step = js[0].w->mw.kind == KIND_Q6K ? 0.9f : nb > 32 ? 0.5f : 0.6f;
     const float token = std::max(nb > 32 ? 0.7f : 0.35f, blocks / 40000.f);
     return 2.7f + blocks / 18000.f + (float)nt * token < 3.3f + (float)steps * step + blocks / 60000.f;
@@ -522,7 +523,7 @@ static bool kq_matvec(const JobSpec* js, int njobs, int nt) {
 
 static bool run_multi(Ctx* c, const JobSpec* js, int njobs, bool pair, int nt, const MvOpts& o) {
     const bool panel = js[0].w->mw.kind == KIND_PANEL;
-    if (nt > (panel ? kGemmMinTokens : kGemmKqMinTokens) && o.pro == PRO_NONE && (panel || !kq_matvec(js, njobs, nt))) {
+    if (nt > (panel ? kGemmMinTokens : kGemmKqMinTokens) && o.pro == PRO_NONE && (panel || !kq_matvec(js, njobs, pair, nt))) {
         GemmLaunch G;
         memset(&G, 0, sizeof G);
         G.njobs = njobs;
